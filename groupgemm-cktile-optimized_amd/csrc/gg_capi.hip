@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -15,6 +16,7 @@
 #include <string>
 #include <vector>
 
+#include "gg_few.h"
 #include "gg_grouped_gemm.h"
 #include "gg_kernel.h"
 
@@ -46,6 +48,7 @@ struct gg_plan {
     bool                small       = false;
     gg::SmallArgs       sargs{};
     gg::SmallTile      *d_small     = nullptr; // [sargs.tiles]
+    int                 few         = -1;      // few-row plans: the instance of gg_few.hip, -1: none
 };
 
 namespace {
@@ -94,12 +97,35 @@ int check_problem(int dtype, int group_num, int64_t n, int64_t k, bool has_outpu
     return GG_OK;
 }
 
-int device_props(hipDeviceProp_t *prop) {
+// Launch facts of the current device, queried from the runtime on the device's first use.
+struct Device {
+    int cus   = 0;
+    int n_xcd = 1;
+};
+constexpr int kMaxDevices = 64;
+
+int current_device(Device *out) {
+    static std::mutex mu;
+    static Device     known[kMaxDevices];
     int        dev = 0;
     hipError_t e   = hipGetDevice(&dev);
-    if (e == hipSuccess)
-        e = hipGetDeviceProperties(prop, dev);
-    return e == hipSuccess ? GG_OK : hip_fail(e, "hipGetDeviceProperties");
+    if (e != hipSuccess)
+        return hip_fail(e, "hipGetDevice");
+    const bool                  keep = dev >= 0 && dev < kMaxDevices;
+    std::lock_guard<std::mutex> lock(mu);
+    Device                      d = keep ? known[dev] : Device{};
+    if (d.cus == 0) {
+        hipDeviceProp_t prop;
+        e = hipGetDeviceProperties(&prop, dev);
+        if (e != hipSuccess)
+            return hip_fail(e, "hipGetDeviceProperties");
+        d.cus   = prop.multiProcessorCount;
+        d.n_xcd = xcd_count(prop);
+        if (keep)
+            known[dev] = d;
+    }
+    *out = d;
+    return GG_OK;
 }
 
 void fill_args(gg_plan *plan, int n_xcd) {
@@ -177,16 +203,16 @@ int choose_splits(int tiles, int k_tiles, int cus) {
 // tile each (1 x 2048 x 7168: 224 tiles of 256 x 256 on 256 CUs, 256 tiles of 256 x 224). The
 // group table is rebuilt for the narrow tile count. GG_NARROW=0 in the environment turns this
 // off.
-int use_narrow_tiles(gg_plan *plan, const int64_t *group_m, const hipDeviceProp_t &prop, hipStream_t s) {
+int use_narrow_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, hipStream_t s) {
     gg::KernelArgs &a   = plan->args;
     const char     *env = std::getenv("GG_NARROW");
     if ((env != nullptr && *env != '\0' && std::atoi(env) == 0) || a.splits > 1 || a.tile_m != gg::kTileM ||
-        plan->total_tiles >= prop.multiProcessorCount)
+        plan->total_tiles >= dev.cus)
         return GG_OK;
     const int64_t               n_tiles = gg::cdiv(plan->n, gg::kNarrowTileN);
     std::vector<gg::GroupEntry> table(static_cast<size_t>(plan->group_num));
     const int64_t tiles = gg::build_group_table(group_m, plan->group_num, n_tiles, table.data());
-    if (tiles <= plan->total_tiles || tiles > prop.multiProcessorCount)
+    if (tiles <= plan->total_tiles || tiles > dev.cus)
         return GG_OK;
     hipError_t e = hipMemcpyAsync(plan->d_groups, table.data(), table.size() * sizeof(gg::GroupEntry),
                                   hipMemcpyHostToDevice, s);
@@ -199,7 +225,7 @@ int use_narrow_tiles(gg_plan *plan, const int64_t *group_m, const hipDeviceProp_
     a.total_tiles     = plan->total_tiles;
     a.n_tiles         = static_cast<int>(n_tiles);
     a.tile_n          = gg::kNarrowTileN;
-    const int n_xcd   = xcd_count(prop);
+    const int n_xcd   = dev.n_xcd;
     a.n_xcd           = plan->grid % n_xcd == 0 ? n_xcd : 1;
     return GG_OK;
 }
@@ -285,7 +311,7 @@ int use_short_tiles(gg_plan *plan, const int64_t *group_m, hipStream_t s) {
 // plan allows them.
 constexpr double kWideTileCost = 1.10;
 
-int use_short_wide_tiles(gg_plan *plan, const int64_t *group_m, const hipDeviceProp_t &prop, hipStream_t s) {
+int use_short_wide_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, hipStream_t s) {
     gg::KernelArgs &a   = plan->args;
     const char     *env = std::getenv("GG_WIDE");
     const int       opt = env != nullptr && *env != '\0' ? std::atoi(env) : -1;
@@ -297,8 +323,8 @@ int use_short_wide_tiles(gg_plan *plan, const int64_t *group_m, const hipDeviceP
     const int64_t tiles = gg::build_group_table(group_m, plan->group_num, n_tiles, table.data(), 0, a.tile_m);
     if (tiles <= 0 || tiles > INT32_MAX)
         return GG_OK;
-    const int grid  = static_cast<int>(std::min<int64_t>(prop.multiProcessorCount, tiles));
-    const int n_xcd = grid % xcd_count(prop) == 0 ? xcd_count(prop) : 1;
+    const int grid  = static_cast<int>(std::min<int64_t>(dev.cus, tiles));
+    const int n_xcd = grid % dev.n_xcd == 0 ? dev.n_xcd : 1;
     gg::KernelArgs w = a;
     w.total_tiles    = static_cast<int>(tiles);
     w.n_tiles        = static_cast<int>(n_tiles);
@@ -327,9 +353,9 @@ int use_short_wide_tiles(gg_plan *plan, const int64_t *group_m, const hipDeviceP
 }
 
 // Picks the plan's split count (plan->args filled, k_tiles set) and allocates the partial sums.
-int setup_split_k(gg_plan *plan, const hipDeviceProp_t &prop) {
+int setup_split_k(gg_plan *plan, const Device &dev) {
     gg::KernelArgs &a  = plan->args;
-    const int       sp = choose_splits(plan->total_tiles, a.k_tiles, prop.multiProcessorCount);
+    const int       sp = choose_splits(plan->total_tiles, a.k_tiles, dev.cus);
     if (sp <= 1)
         return GG_OK;
     const size_t bytes = size_t(sp) * size_t(plan->total_tiles) * 262144;
@@ -338,7 +364,7 @@ int setup_split_k(gg_plan *plan, const hipDeviceProp_t &prop) {
         return hip_fail(e, "split-K workspace allocation");
     a.splits    = sp;
     a.ws        = plan->d_ws;
-    plan->grid  = static_cast<int>(std::min<int64_t>(prop.multiProcessorCount, int64_t(sp) * plan->total_tiles));
+    plan->grid  = static_cast<int>(std::min<int64_t>(dev.cus, int64_t(sp) * plan->total_tiles));
     return GG_OK;
 }
 
@@ -413,10 +439,21 @@ constexpr double kSmallStepUs    = 0.62; // one K step of a 128 x 128 tile, one 
 constexpr double kSmallStepTwoUs = 1.0;  // the same with up to two workgroups per CU
 constexpr double kSmallGain      = 0.85;
 
-int use_small_tiles(gg_plan *plan, const int64_t *group_m, const hipDeviceProp_t &prop, hipStream_t s) {
+// The model: `units` small tiles (times K ranges) of `per` steps each against the persistent plan's
+// tiles, splits and K steps.
+bool small_tiles_win(int64_t units, int per, int tiles, int splits, int k_tiles, int cus) {
+    if (2 * int64_t(tiles) > cus || units > 2 * int64_t(cus))
+        return false;
+    const double big  = kSmallFixedUs + gg::cdiv(k_tiles, splits) * kStepUs +
+                       (splits > 1 ? kSplitUs + double(splits) * tiles * kSlabUs : 0.0);
+    const double step = units <= cus ? kSmallStepUs : kSmallStepTwoUs;
+    return kSmallFixedUs + double(per) * step <= kSmallGain * big;
+}
+
+int use_small_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, hipStream_t s) {
     const char *env = std::getenv("GG_SMALL");
     const int   opt = env != nullptr && *env != '\0' ? std::atoi(env) : -1;
-    const int   cus = prop.multiProcessorCount;
+    const int   cus = dev.cus;
     const gg::KernelArgs &a = plan->args;
     if (opt == 0 || plan->group_num > 32767 || (opt != 1 && (2 * plan->total_tiles > cus || a.tail_splits > 1)))
         return GG_OK;
@@ -440,7 +477,7 @@ int use_small_tiles(gg_plan *plan, const int64_t *group_m, const hipDeviceProp_t
     // XCDs in contiguous runs (xcd_remap), so that the workgroups of one XCD share a few x and w
     // panels in its L2 instead of every XCD reading every w panel.
     // (A grid of whole XCD rows: XCD y takes ceil((tiles - y) / n_xcd) of the list.)
-    if (const int n_xcd = xcd_count(prop); n_xcd > 1) {
+    if (const int n_xcd = dev.n_xcd; n_xcd > 1) {
         const int                  rows = static_cast<int>(gg::cdiv(tiles, n_xcd)) * n_xcd;
         std::vector<gg::SmallTile> dealt(list.size());
         for (int t = 0; t < static_cast<int>(tiles); ++t)
@@ -456,14 +493,8 @@ int use_small_tiles(gg_plan *plan, const int64_t *group_m, const hipDeviceProp_t
     sp            = static_cast<int>(gg::cdiv(k_steps, per)); // no empty K range
     // a 4-step ring while every workgroup has a CU of its own, else a 2-step ring, two per CU
     const int stages = tiles * sp <= cus ? gg::kSmallStagesOne : gg::kSmallStagesTwo;
-    if (opt != 1) {
-        const double big   = kSmallFixedUs + gg::cdiv(a.k_tiles, a.splits) * kStepUs +
-                           (a.splits > 1 ? kSplitUs + double(a.splits) * plan->total_tiles * kSlabUs : 0.0);
-        const double step  = stages == gg::kSmallStagesOne ? kSmallStepUs : kSmallStepTwoUs;
-        const double small = kSmallFixedUs + double(per) * step;
-        if (tiles * sp > 2 * int64_t(cus) || small > kSmallGain * big)
-            return GG_OK;
-    }
+    if (opt != 1 && !small_tiles_win(tiles * sp, per, plan->total_tiles, a.splits, a.k_tiles, cus))
+        return GG_OK;
     // the persistent plan's workspace and descriptors are not used by this launch
     if (plan->d_ws != nullptr)
         (void)hipFree(plan->d_ws);
@@ -510,6 +541,171 @@ void free_plan(gg_plan *plan) {
     if (plan->d_desc != nullptr)
         (void)hipFree(plan->d_desc);
     delete plan;
+}
+
+// Few-row tiles (gg_few.hip) for forward and dgrad plans, 16-bit and fp8, host- and device-size,
+// whose groups have few rows or whose whole problem is small: there the 256 x 256 tiles of the
+// persistent kernel (and the 128 x 128 ones) leave CUs idle or run one long chain of K steps each.
+// Chosen by a launch-time model in microseconds, the lesser instance's time against the plan
+// that would run otherwise, taken at kFewGain of it. Both sides add the parts' squares (the memory
+// traffic, the operands' way into LDS and the chain of K steps overlap, but not fully):
+//   few:   kFewFixedUs + |HBM bytes / kFewHbm, staged bytes / kFewStage, rounds of workgroups x
+//          (chunks per wave x chunk_us + kFewRoundUs)|
+//   other: fixed + |HBM bytes / kOtherHbm, K steps of the busiest workgroup|
+// Fitted to 300 random forward and dgrad problems of 1-64 groups, 1-1000 rows each, N and K
+// 512-14336, bf16 and fp8 (MI355X, each instance and the other plan timed): the choice gives
+// 1.70x over the other plans in the geometric mean (the best instance of each 1.76x) and a loss on
+// none. Examples (us, other -> few): 4 x 256 rows, 512 x 1024 12.3 -> 5.4;
+// 3 x 5 rows, 3328 x 12256 199 -> 56; 3 x 14 rows dgrad, 1208 x 2048 25.6 -> 6.3; 16 x 64 rows,
+// 2048 x 1408 29.5 -> 22.5; left: 8 x 128 rows, 4096 x 7168 100 (few 131). With rows for whole
+// tiles, the staged bytes (each small tile stages its own operands) decide against it.
+// Plans of more than kFewMaxSmallTiles 128 x 128 tiles whose groups average over 64 rows keep them:
+// the few-row tiles ran 0.73-1.28x there (7 of the 300 problems), and the model is no better than that.
+// GG_SMALL in the environment (0: no small tiles, 1: 128 x 128 tiles) turns it off; without it,
+// GG_FEW=<i> takes instance i (GG_FEW=-1: none).
+constexpr double kFewGain = 0.85, kFewFixedUs = 1.6, kFewRoundUs = 1.9;
+constexpr double kFewHbm = 6.2e6, kFewStageFwd = 22e6, kFewStageDgrad16 = 15e6, kFewStageDgrad8 = 10.5e6; // bytes per us
+constexpr int    kFewMaxSmallTiles = 64;
+constexpr double kOtherHbm16 = 6.8e6, kOtherHbm8 = 5.9e6;
+constexpr double kOtherFixedUs = 7.2, kOtherStepUs = 0.88;  // persistent kernel
+constexpr double kOtherSmallFixedUs = 1.8;                  // 128 x 128 tiles
+
+// Row tiles of bm rows: of the host's sizes, or of `rows` rows spread over the groups (device sizes:
+// a group whose average fills more than half a tile is expected to end in half a tile).
+double row_tiles(const int64_t *group_m, int group_num, int64_t rows, int bm) {
+    if (group_m == nullptr) {
+        const double avg = double(rows) / group_num;
+        return std::max(double(std::min<int64_t>(group_num, rows)), double(rows) / bm + (avg > bm / 2 ? 0.5 * group_num : 0.0));
+    }
+    double t = 0;
+    for (int g = 0; g < group_num; ++g)
+        t += static_cast<double>(gg::cdiv(group_m[g], bm));
+    return t;
+}
+
+// The few-row instance of a forward or dgrad plan (its problem set; group_m null: device sizes of
+// `rows` rows in all), or -1.
+int choose_few_rows(const gg_plan *plan, const int64_t *group_m, int64_t rows, int cus) {
+    if (const char *env = std::getenv("GG_SMALL"); env != nullptr && *env != '\0')
+        return -1;
+    int forced = -2;
+    if (const char *env = std::getenv("GG_FEW"); env != nullptr && *env != '\0')
+        forced = std::atoi(env);
+    if (forced == -1 || forced >= gg::kFewInstanceCount)
+        return -1;
+    const bool    f8 = plan->mode / 4 != gg::kIn16, dgrad = plan->mode % 4 == gg::kDgrad;
+    const int     es     = f8 ? 1 : 2;
+    const int64_t groups = std::min<int64_t>(plan->group_num, rows);
+    const int64_t chunks = gg::cdiv(plan->k * es, 128); // 128 bytes of an operand row
+    const double  bytes  = double(groups) * plan->n * plan->k * es + double(rows) * (plan->k * es + plan->n * 2);
+    // the plan that would run otherwise
+    const double tiles = row_tiles(group_m, plan->group_num, rows, gg::kTileM) * gg::cdiv(plan->n, gg::kTileN);
+    double       steps, fixed = kOtherFixedUs;
+    if (group_m == nullptr || tiles > cus) {
+        steps = std::max(1.0, std::ceil(tiles / cus)) * chunks * kOtherStepUs;
+    } else {
+        const int s = choose_splits(static_cast<int>(tiles), static_cast<int>(chunks), cus);
+        steps       = gg::cdiv(chunks, s) * kOtherStepUs + (s > 1 ? kSplitUs + s * tiles * kSlabUs : 0.0);
+        const double units = row_tiles(group_m, plan->group_num, rows, gg::kSmallTile) * gg::cdiv(plan->n, gg::kSmallTile);
+        if (!f8 && !dgrad && small_tiles_win(static_cast<int64_t>(units), static_cast<int>(chunks), static_cast<int>(tiles), s,
+                                             static_cast<int>(chunks), cus)) {
+            if (forced < 0 && units > kFewMaxSmallTiles && rows > 64 * groups)
+                return -1;
+            steps = chunks * (units <= cus ? kSmallStepUs : kSmallStepTwoUs);
+            fixed = kOtherSmallFixedUs;
+        }
+    }
+    const double other = fixed + std::hypot(bytes / (f8 ? kOtherHbm8 : kOtherHbm16), steps);
+    const double stage = !dgrad ? kFewStageFwd : f8 ? kFewStageDgrad8 : kFewStageDgrad16;
+    int          best  = -1;
+    double       least = kFewGain * other;
+    for (int i = 0; i < gg::kFewInstanceCount; ++i) {
+        const gg::FewInstance &f = gg::kFewInstances[i];
+        // (device sizes may put every row in each group: the count must fit 32 bits even then)
+        const int64_t nt = gg::cdiv(plan->n, f.tile_n);
+        if (forced >= 0 ? i != forced
+                        : double(plan->group_num) * double(gg::cdiv(rows, f.tile_m)) * double(nt) > double(INT32_MAX))
+            continue;
+        const double wgs    = row_tiles(group_m, plan->group_num, rows, f.tile_m) * nt;
+        const double staged = wgs * (f.tile_m + f.tile_n) * 128.0 * chunks;
+        const double chain  = std::max(1.0, std::ceil(wgs / (cus * f.per_cu))) * (gg::cdiv(chunks, f.waves) * f.chunk_us + kFewRoundUs);
+        const double us     = kFewFixedUs + std::hypot(bytes / kFewHbm, staged / stage, chain);
+        if (forced >= 0 || us < least) {
+            least = us;
+            best  = i;
+        }
+    }
+    return best;
+}
+
+// The few-row kernel's operand format of a plan.
+int few_format(const gg_plan *plan) {
+    switch (plan->mode / 4) {
+    case gg::kInE4M3: return gg::kFewE4M3;
+    case gg::kInE5M2: return gg::kFewE5M2;
+    case gg::kInE5M2xE4M3: return gg::kFewE5M2xE4M3;
+    default: return plan->dtype == GG_DTYPE_FP16 ? gg::kFewF16 : gg::kFewBF16;
+    }
+}
+
+// The tiles of a few-row plan in its arguments (after fill_args) and its launch: one workgroup per
+// tile of at most `tiles`, in whole XCD rows (a workgroup goes on to further tiles if there are more).
+void few_args(gg_plan *plan, int64_t tiles) {
+    gg::KernelArgs &a = plan->args;
+    a.tile_m          = gg::kFewInstances[plan->few].tile_m;
+    a.tile_n          = gg::kFewInstances[plan->few].tile_n;
+    a.n_tiles         = static_cast<int>(gg::cdiv(plan->n, a.tile_n));
+    a.d_total         = nullptr;
+    if (plan->mode % 4 == gg::kDgrad) {
+        a.lda = static_cast<int>(plan->k);
+        a.ldb = static_cast<int>(plan->n);
+    }
+    plan->grid = static_cast<int>(gg::cdiv(std::min<int64_t>(tiles, 1 << 20), 8) * 8);
+}
+
+std::string few_detail(const gg_plan *plan, const std::string &what) {
+    return "mi355x few-row " + std::to_string(plan->args.tile_m) + "x" + std::to_string(plan->args.tile_n) + " " + what +
+           " grid=" + std::to_string(plan->grid) +
+           (plan->device_lens ? std::string(plan->in_kernel_table ? " tiles=device (device group sizes, in-kernel table)"
+                                                                  : " tiles=device (device group sizes)")
+                              : " tiles=" + std::to_string(plan->total_tiles));
+}
+
+// Turns a host-size forward or dgrad plan (its problem set) into a few-row plan where
+// choose_few_rows takes one: the group table of the instance's tiles and the launch.
+int use_few_rows(gg_plan *plan, const int64_t *group_m, const float *x_scale, const float *w_scale,
+                 const std::string &what, hipStream_t s) {
+    Device dev;
+    if (current_device(&dev) != GG_OK)
+        return GG_ERR_HIP;
+    const int few = choose_few_rows(plan, group_m, plan->total_m, dev.cus);
+    if (few < 0)
+        return GG_OK;
+    const gg::FewInstance      &f = gg::kFewInstances[few];
+    std::vector<gg::GroupEntry> table(static_cast<size_t>(plan->group_num));
+    const int64_t tiles = gg::build_group_table(group_m, plan->group_num, gg::cdiv(plan->n, f.tile_n), table.data(), 0, f.tile_m);
+    if (tiles <= 0)
+        return GG_OK;
+    const size_t bytes = table.size() * sizeof(gg::GroupEntry);
+    hipError_t   e     = hipMalloc(&plan->d_groups, bytes);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(plan->d_groups, table.data(), bytes, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(s);
+    if (e != hipSuccess)
+        return hip_fail(e, "few-row group table");
+    plan->few         = few;
+    plan->total_tiles = static_cast<int>(tiles);
+    plan->grid        = 0;
+    fill_args(plan, 1);
+    few_args(plan, tiles);
+    const int n_xcd        = dev.n_xcd;
+    plan->args.n_xcd       = plan->grid % n_xcd == 0 ? n_xcd : 1;
+    plan->args.total_tiles = plan->total_tiles;
+    plan->args.x_scale     = x_scale;
+    plan->args.w_scale     = w_scale;
+    plan->detail           = few_detail(plan, what);
+    return GG_OK;
 }
 
 // Tile descriptors of forward, dgrad and wgrad plans of whole tiles (host-size tables): every
@@ -585,50 +781,34 @@ namespace {
 // header. One copy per GPU, held until the process ends; every call on a GPU shares it, so
 // calls that overlap on one GPU (two streams, two host threads) race on it. Host code never
 // names `scratch` in a kernel argument or copy: it uses the device address that
-// hipGetSymbolAddress gives for the current device (noalloc_device).
+// hipGetSymbolAddress gives for the current device (noalloc_scratch).
 constexpr int    kNoAllocMaxGroups  = 8192;
 constexpr size_t kNoAllocTableBytes = size_t(kNoAllocMaxGroups) * sizeof(gg::GroupEntry);
 constexpr size_t kScratchBytes      = kNoAllocTableBytes + 256; // + the TableHeader, padded
 static_assert(sizeof(gg::TableHeader) <= 256, "the header fits behind the largest table");
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-// What the allocation-free entry point keeps per device: the scratch address and the launch
-// facts of hipGetDeviceProperties (queried once, not per call).
-struct NoAllocDevice {
-    void *scratch = nullptr;
-    int   cus     = 0;
-    int   n_xcd   = 1;
-};
-constexpr int kNoAllocMaxDevices = 64;
-std::mutex    g_noalloc_mu;
-NoAllocDevice g_noalloc_dev[kNoAllocMaxDevices];
-
-// The current device's entry, set up on its first use with that device current.
-int noalloc_device(NoAllocDevice *out) {
+// The current device's scratch address, looked up on its first use with that device current.
+int noalloc_scratch(void **out) {
+    static std::mutex mu;
+    static void      *known[kMaxDevices];
     int        dev = 0;
     hipError_t e   = hipGetDevice(&dev);
     if (e != hipSuccess)
         return hip_fail(e, "hipGetDevice");
-    if (dev < 0 || dev >= kNoAllocMaxDevices)
-        return fail(GG_ERR_UNSUPPORTED, "device index " + std::to_string(dev) + " beyond " +
-                                            std::to_string(kNoAllocMaxDevices));
-    std::lock_guard<std::mutex> lock(g_noalloc_mu);
-    NoAllocDevice              &d = g_noalloc_dev[dev];
-    if (d.scratch == nullptr) {
-        hipDeviceProp_t prop;
-        if (device_props(&prop) != GG_OK)
-            return GG_ERR_HIP;
+    if (dev < 0 || dev >= kMaxDevices)
+        return fail(GG_ERR_UNSUPPORTED, "device index " + std::to_string(dev) + " beyond " + std::to_string(kMaxDevices));
+    std::lock_guard<std::mutex> lock(mu);
+    if (known[dev] == nullptr) {
         void *p = nullptr;
         e       = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess)
             return hip_fail(e, "hipGetSymbolAddress(scratch)");
         if (p == nullptr || (reinterpret_cast<uintptr_t>(p) & 255u) != 0)
             return fail(GG_ERR_HIP, "hipGetSymbolAddress(scratch) gave a null or misaligned address");
-        d.cus     = prop.multiProcessorCount;
-        d.n_xcd   = xcd_count(prop);
-        d.scratch = p;
+        known[dev] = p;
     }
-    *out = d;
+    *out = known[dev];
     return GG_OK;
 }
 
@@ -731,22 +911,18 @@ int plan_device_lens(gg_plan *plan, bool noalloc, int op, int a_dtype, int b_dty
             plan->total_m = 0;
         return GG_OK;
     }
-    int cus = 0, n_xcd = 1;
     const size_t table_bytes = static_cast<size_t>(group_num) * sizeof(gg::GroupEntry);
+    Device       dev;
+    if (const int st = current_device(&dev); st != GG_OK)
+        return st;
+    const int cus = dev.cus, n_xcd = dev.n_xcd;
     if (noalloc) {
-        NoAllocDevice d;
-        if (const int st = noalloc_device(&d); st != GG_OK)
+        void *mem = nullptr;
+        if (const int st = noalloc_scratch(&mem); st != GG_OK)
             return st;
-        cus            = d.cus;
-        n_xcd          = d.n_xcd;
-        plan->d_groups = static_cast<gg::GroupEntry *>(d.scratch);
-        plan->d_header = reinterpret_cast<gg::TableHeader *>(static_cast<char *>(d.scratch) + kNoAllocTableBytes);
+        plan->d_groups = static_cast<gg::GroupEntry *>(mem);
+        plan->d_header = reinterpret_cast<gg::TableHeader *>(static_cast<char *>(mem) + kNoAllocTableBytes);
     } else {
-        hipDeviceProp_t prop;
-        if (device_props(&prop) != GG_OK)
-            return GG_ERR_HIP;
-        cus   = prop.multiProcessorCount;
-        n_xcd = xcd_count(prop);
         // Table + header in one allocation; the header is written by every run.
         const hipError_t e = hipMalloc(&plan->d_groups, table_bytes + sizeof(gg::TableHeader));
         if (e != hipSuccess) {
@@ -770,7 +946,14 @@ int plan_device_lens(gg_plan *plan, bool noalloc, int op, int a_dtype, int b_dty
         ka.lda = static_cast<int>(n);
         ka.ldb = static_cast<int>(k);
     }
-    if (op == GG_OP_WGRAD) {
+    if (op != GG_OP_WGRAD)
+        plan->few = choose_few_rows(plan, nullptr, total_m, cus);
+    if (plan->few >= 0) {
+        const gg::FewInstance &f = gg::kFewInstances[plan->few];
+        few_args(plan, (total_m / f.tile_m + std::min<int64_t>(group_num, total_m)) * gg::cdiv(n_out, f.tile_n));
+        ka.total_tiles = 0;
+        ka.d_total     = &plan->d_header->run_tiles;
+    } else if (op == GG_OP_WGRAD) {
         // The K-step counts depend on the sizes; a cross-tile wgrad tile runs at least
         // kCrossMinStepsHost of them (zeros past its group's rows), so the cross-tile variant runs.
         ka.m_out          = static_cast<int>(n);
@@ -803,7 +986,9 @@ int plan_device_lens(gg_plan *plan, bool noalloc, int op, int a_dtype, int b_dty
         ka.d_total            = nullptr;
     }
     ka.n_xcd = plan->grid % n_xcd == 0 ? n_xcd : 1;
-    if (!noalloc)
+    if (!noalloc && plan->few >= 0)
+        plan->detail = few_detail(plan, what);
+    else if (!noalloc)
         plan->detail = "mi355x " + what + " persistent 256x256x" + std::to_string(f8 ? 128 : 64) + " grid=" +
                        std::to_string(plan->grid) + " tiles=" +
                        (op == GG_OP_WGRAD ? std::to_string(plan->total_tiles) : std::string("device")) +
@@ -812,6 +997,11 @@ int plan_device_lens(gg_plan *plan, bool noalloc, int op, int a_dtype, int b_dty
                        (ka.band != gg::kBand ? " band=" + std::to_string(ka.band) : "") +
                        (plan->in_kernel_table ? " (device group sizes, in-kernel table)" : " (device group sizes)");
     return GG_OK;
+}
+
+int run_few(const gg_plan *plan, hipStream_t s) {
+    const hipError_t e = gg::launch_few_gemm(plan->args, few_format(plan), plan->mode % 4 == gg::kDgrad, plan->few, plan->grid, s);
+    return e == hipSuccess ? GG_OK : hip_fail(e, "few-row GEMM launch");
 }
 
 // Enqueue a plan's launches on `stream` (gg_run). zero_kernel: an empty contraction zero-fills
@@ -824,10 +1014,13 @@ int run_plan(const gg_plan *plan, void *stream, bool zero_kernel) {
         if (!plan->in_kernel_table) {
             e = gg::launch_build_group_table(plan->d_lens, plan->d_offs, plan->group_num, plan->in_rows,
                                              plan->args.n_tiles, plan->d_groups, plan->d_header, s,
-                                             plan->args.m_out);
+                                             plan->args.m_out, plan->args.tile_m,
+                                             plan->few >= 0 ? static_cast<int>(gg::cdiv(plan->n, gg::kTileN)) : 0);
             if (e != hipSuccess)
                 return hip_fail(e, "group table launch");
         }
+        if (plan->few >= 0)
+            return run_few(plan, s);
         e = gg::launch_grouped_gemm(plan->args, plan->dtype == GG_DTYPE_FP16, plan->grid, s, plan->mode);
         if (e != hipSuccess)
             return hip_fail(e, "grouped GEMM launch");
@@ -844,6 +1037,8 @@ int run_plan(const gg_plan *plan, void *stream, bool zero_kernel) {
         }
         return GG_OK;
     }
+    if (plan->few >= 0)
+        return run_few(plan, s);
     if (plan->small) {
         const hipError_t e = gg::launch_small_gemm(plan->sargs, plan->dtype == GG_DTYPE_FP16, s);
         return e == hipSuccess ? GG_OK : hip_fail(e, "small-tile GEMM launch");
@@ -913,8 +1108,18 @@ int gg_prepare(int dtype, int group_num, int64_t n, int64_t k, const int64_t *gr
 
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (plan->total_tiles > 0) {
-        hipDeviceProp_t prop;
-        if (device_props(&prop) != GG_OK) {
+        if (use_few_rows(plan, group_m, nullptr, nullptr, dtype == GG_DTYPE_BF16 ? "bf16" : "fp16", s) != GG_OK) {
+            free_plan(plan);
+            return GG_ERR_HIP;
+        }
+        if (plan->few >= 0) {
+            *plan_out = plan;
+            return GG_OK;
+        }
+    }
+    if (plan->total_tiles > 0) {
+        Device dev;
+        if (current_device(&dev) != GG_OK) {
             delete plan;
             return GG_ERR_HIP;
         }
@@ -931,13 +1136,13 @@ int gg_prepare(int dtype, int group_num, int64_t n, int64_t k, const int64_t *gr
             return hip_fail(e, "group table upload");
         }
         // Persistent grid: one workgroup per CU (160 KB of LDS each), never more than tiles.
-        plan->grid = std::min(prop.multiProcessorCount, plan->total_tiles);
-        fill_args(plan, xcd_count(prop));
+        plan->grid = std::min(dev.cus, plan->total_tiles);
+        fill_args(plan, dev.n_xcd);
         gg::KernelArgs &a = plan->args;
         a.total_tiles     = plan->total_tiles;
         a.d_total         = nullptr;
         a.tails           = k % gg::kTileK != 0; // K-major operands: only a partial K step
-        if (setup_split_k(plan, prop) != GG_OK) {
+        if (setup_split_k(plan, dev) != GG_OK) {
             free_plan(plan);
             return GG_ERR_HIP;
         }
@@ -945,11 +1150,11 @@ int gg_prepare(int dtype, int group_num, int64_t n, int64_t k, const int64_t *gr
             free_plan(plan);
             return st2;
         }
-        if (use_short_wide_tiles(plan, group_m, prop, s) != GG_OK) {
+        if (use_short_wide_tiles(plan, group_m, dev, s) != GG_OK) {
             free_plan(plan);
             return GG_ERR_HIP;
         }
-        if (use_narrow_tiles(plan, group_m, prop, s) != GG_OK) {
+        if (use_narrow_tiles(plan, group_m, dev, s) != GG_OK) {
             free_plan(plan);
             return GG_ERR_HIP;
         }
@@ -961,7 +1166,7 @@ int gg_prepare(int dtype, int group_num, int64_t n, int64_t k, const int64_t *gr
             free_plan(plan);
             return st3;
         }
-        if (const int st4 = use_small_tiles(plan, group_m, prop, s); st4 != GG_OK) {
+        if (const int st4 = use_small_tiles(plan, group_m, dev, s); st4 != GG_OK) {
             free_plan(plan);
             return st4;
         }
@@ -1087,9 +1292,20 @@ static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num,
                               : format == gg::kInE4M3     ? " fp8 e4m3"
                               : format == gg::kInE5M2     ? " fp8 e5m2"
                                                           : " fp8 e5m2 x e4m3");
+    if (plan->total_tiles > 0 && dgrad) {
+        const std::string in = f8 ? "" : dtype_a == GG_DTYPE_BF16 ? " bf16" : " fp16";
+        if (use_few_rows(plan, group_m, f8 ? a_scale : nullptr, f8 ? b_scale : nullptr, what + in, s) != GG_OK) {
+            free_plan(plan);
+            return GG_ERR_HIP;
+        }
+        if (plan->few >= 0) {
+            *plan_out = plan;
+            return GG_OK;
+        }
+    }
     if (plan->total_tiles > 0) {
-        hipDeviceProp_t prop;
-        if (device_props(&prop) != GG_OK) {
+        Device dev;
+        if (current_device(&dev) != GG_OK) {
             delete plan;
             return GG_ERR_HIP;
         }
@@ -1105,8 +1321,8 @@ static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num,
             delete plan;
             return hip_fail(e, "group table upload");
         }
-        plan->grid = std::min(prop.multiProcessorCount, plan->total_tiles);
-        fill_args(plan, xcd_count(prop));
+        plan->grid = std::min(dev.cus, plan->total_tiles);
+        fill_args(plan, dev.n_xcd);
         gg::KernelArgs &ka = plan->args;
         ka.total_tiles     = plan->total_tiles;
         ka.d_total         = nullptr;
@@ -1130,7 +1346,7 @@ static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num,
             ka.tails = t;
         }
         // wgrad's K steps differ per group: no split
-        if (dgrad && setup_split_k(plan, prop) != GG_OK) {
+        if (dgrad && setup_split_k(plan, dev) != GG_OK) {
             free_plan(plan);
             return GG_ERR_HIP;
         }
@@ -1218,8 +1434,18 @@ int gg_prepare_fp8(int dtype, int group_num, int64_t n, int64_t k, const int64_t
     plan->total_tiles = has_output && k > 0 ? static_cast<int>(tiles) : 0;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (plan->total_tiles > 0) {
-        hipDeviceProp_t prop;
-        if (device_props(&prop) != GG_OK) {
+        if (use_few_rows(plan, group_m, x_scale, w_scale, dtype == GG_DTYPE_FP8_E4M3 ? "fp8 e4m3" : "fp8 e5m2", s) != GG_OK) {
+            free_plan(plan);
+            return GG_ERR_HIP;
+        }
+        if (plan->few >= 0) {
+            *plan_out = plan;
+            return GG_OK;
+        }
+    }
+    if (plan->total_tiles > 0) {
+        Device dev;
+        if (current_device(&dev) != GG_OK) {
             delete plan;
             return GG_ERR_HIP;
         }
@@ -1235,8 +1461,8 @@ int gg_prepare_fp8(int dtype, int group_num, int64_t n, int64_t k, const int64_t
             delete plan;
             return hip_fail(e, "group table upload");
         }
-        plan->grid = std::min(prop.multiProcessorCount, plan->total_tiles);
-        fill_args(plan, xcd_count(prop));
+        plan->grid = std::min(dev.cus, plan->total_tiles);
+        fill_args(plan, dev.n_xcd);
         gg::KernelArgs &a = plan->args;
         a.total_tiles     = plan->total_tiles;
         a.d_total         = nullptr;
@@ -1244,7 +1470,7 @@ int gg_prepare_fp8(int dtype, int group_num, int64_t n, int64_t k, const int64_t
         a.tails           = k % 128 != 0;
         a.x_scale         = x_scale;
         a.w_scale         = w_scale;
-        if (setup_split_k(plan, prop) != GG_OK) {
+        if (setup_split_k(plan, dev) != GG_OK) {
             free_plan(plan);
             return GG_ERR_HIP;
         }

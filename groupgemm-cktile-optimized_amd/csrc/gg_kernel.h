@@ -21,10 +21,10 @@ constexpr int make_mode(int layout, int format) { return layout + 4 * format; }
 
 // Header of a device-built group table (follows the group_num entries).
 struct TableHeader {
-    int total_tiles; // tiles over all groups (0 if the count overflowed)
+    int total_tiles; // 256 x 256 tiles over all groups (0 if the count overflowed)
     int first_bad;   // first group whose length or offset was out of range, -1 if none
     int overflow;    // 1 if the tile count exceeded 32 bits (nothing is computed then)
-    int reserved;
+    int run_tiles;   // the table kernel's own tile count (0 where the GEMM builds the table)
 };
 
 // Device-resident group sizes of at most this many groups: the grouped GEMM builds the group
@@ -147,9 +147,12 @@ hipError_t launch_tail_reduce(const KernelArgs &args, bool fp16, int grid, hipSt
 // (int64 rows) and offs[group_num + 1] (int64 first rows) or null for back-to-back groups.
 // Groups outside [0, total_m) get no rows (forward / dgrad: no tiles) and are reported in the
 // header. out_rows > 0 (wgrad): every group owns ceil(out_rows / 256) * n_tiles tiles. One wave.
+// tile_m, n_tiles: the table's tiles. wide_n_tiles > 0: the header's total_tiles counts 256-row
+// tiles times it (a table of other tiles than 256 x 256, whose count goes to run_tiles).
 hipError_t launch_build_group_table(const int64_t *lens, const int64_t *offs, int group_num,
                                     int64_t total_m, int n_tiles, GroupEntry *table,
-                                    TableHeader *header, hipStream_t stream, int out_rows = 0);
+                                    TableHeader *header, hipStream_t stream, int out_rows = 0,
+                                    int tile_m = kTileM, int wide_n_tiles = 0);
 
 // offs[0] = 0, offs[g + 1] = offs[g] + lens[g]: group offsets from device lengths. One wave.
 hipError_t launch_group_offsets(const int64_t *lens, int64_t *offs, int group_num, hipStream_t stream);

@@ -87,9 +87,10 @@ __global__ void __launch_bounds__(256) tail_reduce_kernel(const KernelArgs args,
 // ---------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(64)
 build_group_table_kernel(const int64_t *lens, const int64_t *offs, int group_num, int64_t total_m,
-                         int n_tiles, GroupEntry *table, TableHeader *header, int out_rows) {
+                         int n_tiles, GroupEntry *table, TableHeader *header, int out_rows, int tile_m,
+                         int wide_n_tiles) {
     const int lane      = threadIdx.x;
-    int64_t   row_carry = 0, tile_carry = 0;
+    int64_t   row_carry = 0, tile_carry = 0, wide_carry = 0;
     int       first_bad = -1;
     for (int base = 0; base < group_num; base += 64) {
         const int g     = base + lane;
@@ -103,9 +104,10 @@ build_group_table_kernel(const int64_t *lens, const int64_t *offs, int group_num
         ok = ok && row0 >= 0 && row0 <= total_m && m <= total_m - row0;
         // wgrad (out_rows > 0): every group owns the tiles of its out_rows x N output, zero
         // for a group without rows or with sizes that do not fit
-        const int64_t tiles      = out_rows > 0 ? (live ? cdiv(out_rows, kTileM) * n_tiles : 0)
-                                                : (ok ? cdiv(m, kTileM) * n_tiles : 0);
+        const int64_t tiles      = out_rows > 0 ? (live ? cdiv(out_rows, tile_m) * n_tiles : 0)
+                                                : (ok ? cdiv(m, tile_m) * n_tiles : 0);
         const int64_t tiles_incl = wave_inclusive_sum(tiles, lane);
+        const int64_t wide       = wave_inclusive_sum(ok ? cdiv(m, kTileM) * wide_n_tiles : 0, lane);
         if (live) {
             GroupEntry e;
             e.row0   = ok ? row0 : 0;
@@ -118,13 +120,17 @@ build_group_table_kernel(const int64_t *lens, const int64_t *offs, int group_num
             first_bad = base + __builtin_ctzll(bad);
         row_carry += __shfl(rows_incl, 63, 64);
         tile_carry += __shfl(tiles_incl, 63, 64);
+        wide_carry += __shfl(wide, 63, 64);
     }
     if (lane == 0) {
-        const bool over     = tile_carry > INT32_MAX;
-        header->total_tiles = over ? 0 : static_cast<int>(tile_carry);
+        // the header counts 256 x 256 tiles whatever kernel runs; a kernel of other tiles
+        // (wide_n_tiles > 0) reads its own count from run_tiles
+        const int64_t count = wide_n_tiles > 0 ? wide_carry : tile_carry;
+        const bool    over  = tile_carry > INT32_MAX || count > INT32_MAX;
+        header->total_tiles = over ? 0 : static_cast<int>(count);
         header->first_bad   = first_bad;
         header->overflow    = over ? 1 : 0;
-        header->reserved    = 0;
+        header->run_tiles   = over ? 0 : static_cast<int>(tile_carry);
     }
 }
 
@@ -308,9 +314,10 @@ hipError_t launch_split_reduce(const KernelArgs &args, bool fp16, hipStream_t st
 
 hipError_t launch_build_group_table(const int64_t *lens, const int64_t *offs, int group_num,
                                     int64_t total_m, int n_tiles, GroupEntry *table,
-                                    TableHeader *header, hipStream_t stream, int out_rows) {
+                                    TableHeader *header, hipStream_t stream, int out_rows, int tile_m,
+                                    int wide_n_tiles) {
     hipLaunchKernelGGL(build_group_table_kernel, dim3(1), dim3(64), 0, stream, lens, offs,
-                       group_num, total_m, n_tiles, table, header, out_rows);
+                       group_num, total_m, n_tiles, table, header, out_rows, tile_m, wide_n_tiles);
     return hipGetLastError();
 }
 

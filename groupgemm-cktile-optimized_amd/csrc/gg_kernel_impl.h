@@ -859,7 +859,8 @@ struct LaneGroup {
 // it exceeds 32 bits; *first_bad the first invalid group or -1.
 __device__ __forceinline__ LaneGroup lane_group_table(const int64_t *lens, const int64_t *offs, int group_num,
                                                       int64_t total_m, int n_tiles, int out_rows, int lane,
-                                                      int *total, int *first_bad, int *overflow) {
+                                                      int *total, int *first_bad, int *overflow,
+                                                      int tile_m = kTileM) {
     const bool live = lane < group_num;
     int64_t    m    = live ? lens[lane] : 0;
     bool       ok   = m >= 0 && m <= INT32_MAX;
@@ -868,8 +869,8 @@ __device__ __forceinline__ LaneGroup lane_group_table(const int64_t *lens, const
     const int64_t rows_incl = wave_inclusive_sum(m, lane);
     const int64_t row0      = offs != nullptr ? (live ? offs[lane] : 0) : rows_incl - m;
     ok                      = ok && row0 >= 0 && row0 <= total_m && m <= total_m - row0;
-    const int64_t tiles     = out_rows > 0 ? (live ? cdiv(out_rows, kTileM) * n_tiles : 0)
-                                           : (ok ? cdiv(m, kTileM) * n_tiles : 0);
+    const int64_t tiles     = out_rows > 0 ? (live ? cdiv(out_rows, tile_m) * n_tiles : 0)
+                                           : (ok ? cdiv(m, tile_m) * n_tiles : 0);
     const int64_t tiles_incl = wave_inclusive_sum(tiles, lane);
     // the total from lane 63, read into scalar registers (a shuffle would leave it in a VGPR and
     // every value derived from it, the tile loop's bounds included, with it)
@@ -1057,7 +1058,7 @@ grouped_gemm_kernel(const KernelArgs args) {
             args.d_header->total_tiles = lg_total;
             args.d_header->first_bad   = first_bad;
             args.d_header->overflow    = overflow;
-            args.d_header->reserved    = 0;
+            args.d_header->run_tiles   = 0;
         }
     }
     // Tile count: from the kernel arguments, or from a group table built on the device.

@@ -105,12 +105,13 @@ def mean_after_first(ds, key):
     return sum(vals) / len(vals) if vals else None
 
 
-# The GEMM launch of a plan: the persistent kernel, or the small-tile kernel (gg_small.hip).
-GEMM_KERNEL = re.compile(r"(?:grouped_gemm_kernel|small_gemm_kernel)<[^>]*>")
+# The GEMM launch of a plan: the persistent kernel, the small-tile kernel (gg_small.hip) or the
+# few-row kernel (gg_few.hip).
+GEMM_KERNEL = re.compile(r"(?:grouped_gemm_kernel|small_gemm_kernel|few_gemm_kernel)<[^>]*>")
 
 
 def is_gemm(name: str) -> bool:
-    return "grouped_gemm_kernel" in name or "small_gemm_kernel" in name
+    return any(k in name for k in ("grouped_gemm_kernel", "small_gemm_kernel", "few_gemm_kernel"))
 
 
 def instance(name: str) -> str:

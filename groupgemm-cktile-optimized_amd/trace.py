@@ -39,8 +39,9 @@ def log(msg: str) -> None:
     print(f"[trace {time.strftime('%H:%M:%S')}] {msg}", flush=True)
 
 
-# The GEMM launch of a plan: the persistent kernel, or the small-tile kernel (gg_small.hip).
-GEMM_KERNEL = re.compile(r"(grouped_gemm_kernel|small_gemm_kernel)<([^>]*)>")
+# The GEMM launch of a plan: the persistent kernel, the small-tile kernel (gg_small.hip) or the
+# few-row kernel (gg_few.hip).
+GEMM_KERNEL = re.compile(r"(grouped_gemm_kernel|small_gemm_kernel|few_gemm_kernel)<([^>]*)>")
 
 
 def mangled_instance(name: str) -> str:
