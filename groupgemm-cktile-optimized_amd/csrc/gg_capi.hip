@@ -49,6 +49,7 @@ struct gg_plan {
     gg::SmallArgs       sargs{};
     gg::SmallTile      *d_small     = nullptr; // [sargs.tiles]
     int                 few         = -1;      // few-row plans: the instance of gg_few.hip, -1: none
+    bool                wgrad_few   = false;   // wgrad plans: the kernel of gg_wfew.hip
 };
 
 namespace {
@@ -671,6 +672,67 @@ std::string few_detail(const gg_plan *plan, const std::string &what) {
                               : " tiles=" + std::to_string(plan->total_tiles));
 }
 
+// 128 x 128 tiles (gg_wfew.hip) for wgrad plans whose groups have few rows: the persistent kernel
+// runs at least four K steps per 256 x 256 tile and stores it 8 bytes per lane and row, this one
+// runs the chunks there are and stores whole rows. Chosen by a launch-time model in microseconds,
+// taken at kWgradFewGain of the persistent plan's time (|a, b| = sqrt(a^2 + b^2)):
+//   few:        kWgradFewFixedUs + |bytes / kWgradFewHbm,
+//                                   tiles per CU x tile + chunks x |one chunk's latency, tiles per CU x chunk||
+//   persistent: kWgradFixedUs + |bytes / kWgradHbm, rounds x (tile + max(4, K steps) x step)|
+// with the groups' average K steps. Fitted to 320 random problems of 1-64 groups, 1-8000 rows each,
+// n and k 512-14336, bf16 and fp8 (MI355X, both kernels timed): the choice gives 1.41x over the
+// persistent kernel in the geometric mean, 0.95-0.99x on three problems and no loss elsewhere. Up to
+// 64 rows per group 1.8x, 65-256 1.5x; above 500 rows it pays where 256 x 256 tiles leave CUs idle (1.3x)
+// and loses elsewhere (0.7-0.9x: a 64 x 64 quarter per wave reads twice the LDS bytes per MFMA of the
+// persistent kernel's 128 x 128).
+// GG_SMALL in the environment turns it off; without it, GG_WFEW=1 takes it and GG_WFEW=0 does not.
+constexpr double kWgradFewGain = 0.9, kWgradFewFixedUs = 3.7, kWgradFixedUs = 7.8; // us
+constexpr double kWgradFewHbm = 6.1e6, kWgradHbm = 5.1e6;                          // bytes per us
+
+bool choose_wgrad_few(const gg_plan *plan, const int64_t *group_m, int64_t m_out, int64_t rows, int cus) {
+    if (const char *env = std::getenv("GG_SMALL"); env != nullptr && *env != '\0')
+        return false;
+    const double tiles = double(plan->group_num) * gg::cdiv(m_out, gg::kWgradFewTile) * gg::cdiv(plan->n, gg::kWgradFewTile);
+    if (tiles > INT32_MAX - 64)
+        return false;
+    if (const char *env = std::getenv("GG_WFEW"); env != nullptr && *env != '\0')
+        return std::atoi(env) != 0;
+    const bool f8      = plan->mode / 4 != gg::kIn16;
+    const int  es      = f8 ? 1 : 2;
+    const auto average = [&](int rows_per, double least) { // K steps of a group
+        if (group_m == nullptr)
+            return std::max(least, double(rows) / plan->group_num / rows_per + 0.5);
+        double sum = 0;
+        for (int g = 0; g < plan->group_num; ++g)
+            sum += std::max(least, static_cast<double>(gg::cdiv(group_m[g], rows_per)));
+        return sum / plan->group_num;
+    };
+    const double bytes  = double(plan->group_num) * m_out * plan->n * 2 + double(rows) * (m_out + plan->n) * es;
+    const double wide   = double(plan->group_num) * gg::cdiv(m_out, gg::kTileM) * gg::cdiv(plan->n, gg::kTileN);
+    const double steps  = average(f8 ? 128 : 64, gg::kCrossMinStepsHost);
+    const double chunks = average(f8 ? 128 : 32, 0.0);
+    const double per_cu = std::max(0.25, tiles / cus);
+    const double other  = kWgradFixedUs + std::hypot(bytes / kWgradHbm, std::ceil(wide / cus) *
+                                                                           (f8 ? 1.75 + 1.2 * steps : 2.1 + 1.14 * steps));
+    const double few    = kWgradFewFixedUs +
+                       std::hypot(bytes / kWgradFewHbm, f8 ? 0.05 * per_cu + chunks * std::hypot(0.98, 0.55 * per_cu)
+                                                           : 0.32 * per_cu + chunks * std::hypot(0.43, 0.24 * per_cu));
+    return few < kWgradFewGain * other;
+}
+
+// The launch of such a plan, one workgroup per tile in whole XCD rows (after fill_args; m_out: the
+// rows of a group's gradient).
+void wgrad_few_args(gg_plan *plan, int64_t m_out, int n_xcd) {
+    gg::KernelArgs &a = plan->args;
+    a.total_tiles     = static_cast<int>(int64_t(plan->group_num) * gg::cdiv(m_out, gg::kWgradFewTile) *
+                                         gg::cdiv(plan->n, gg::kWgradFewTile));
+    a.m_out           = static_cast<int>(m_out);
+    a.d_total         = nullptr;
+    plan->wgrad_few   = true;
+    plan->grid        = static_cast<int>(gg::cdiv(a.total_tiles, 8) * 8);
+    a.n_xcd           = plan->grid % n_xcd == 0 ? n_xcd : 1;
+}
+
 // Turns a host-size forward or dgrad plan (its problem set) into a few-row plan where
 // choose_few_rows takes one: the group table of the instance's tiles and the launch.
 int use_few_rows(gg_plan *plan, const int64_t *group_m, const float *x_scale, const float *w_scale,
@@ -986,7 +1048,13 @@ int plan_device_lens(gg_plan *plan, bool noalloc, int op, int a_dtype, int b_dty
         ka.d_total            = nullptr;
     }
     ka.n_xcd = plan->grid % n_xcd == 0 ? n_xcd : 1;
-    if (!noalloc && plan->few >= 0)
+    if (op == GG_OP_WGRAD && choose_wgrad_few(plan, nullptr, n, total_m, cus))
+        wgrad_few_args(plan, n, n_xcd);
+    if (!noalloc && plan->wgrad_few)
+        plan->detail = "mi355x " + what + " few-row 128x128 grid=" + std::to_string(plan->grid) + " tiles=" +
+                       std::to_string(ka.total_tiles) +
+                       (plan->in_kernel_table ? " (device group sizes, in-kernel table)" : " (device group sizes)");
+    else if (!noalloc && plan->few >= 0)
         plan->detail = few_detail(plan, what);
     else if (!noalloc)
         plan->detail = "mi355x " + what + " persistent 256x256x" + std::to_string(f8 ? 128 : 64) + " grid=" +
@@ -1000,7 +1068,7 @@ int plan_device_lens(gg_plan *plan, bool noalloc, int op, int a_dtype, int b_dty
 }
 
 int run_few(const gg_plan *plan, hipStream_t s) {
-    const hipError_t e = gg::launch_few_gemm(plan->args, few_format(plan), plan->mode % 4 == gg::kDgrad, plan->few, plan->grid, s);
+    const hipError_t e = plan->wgrad_few ? gg::launch_wgrad_few(plan->args, few_format(plan), plan->grid, s) : gg::launch_few_gemm(plan->args, few_format(plan), plan->mode % 4 == gg::kDgrad, plan->few, plan->grid, s);
     return e == hipSuccess ? GG_OK : hip_fail(e, "few-row GEMM launch");
 }
 
@@ -1019,7 +1087,7 @@ int run_plan(const gg_plan *plan, void *stream, bool zero_kernel) {
             if (e != hipSuccess)
                 return hip_fail(e, "group table launch");
         }
-        if (plan->few >= 0)
+        if (plan->few >= 0 || plan->wgrad_few)
             return run_few(plan, s);
         e = gg::launch_grouped_gemm(plan->args, plan->dtype == GG_DTYPE_FP16, plan->grid, s, plan->mode);
         if (e != hipSuccess)
@@ -1037,7 +1105,7 @@ int run_plan(const gg_plan *plan, void *stream, bool zero_kernel) {
         }
         return GG_OK;
     }
-    if (plan->few >= 0)
+    if (plan->few >= 0 || plan->wgrad_few)
         return run_few(plan, s);
     if (plan->small) {
         const hipError_t e = gg::launch_small_gemm(plan->sargs, plan->dtype == GG_DTYPE_FP16, s);
@@ -1344,6 +1412,14 @@ static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num,
             for (int g = 0; g < group_num; ++g)
                 t = t || group_m[g] % steps != 0 || group_m[g] < gg::kCrossMinStepsHost * steps;
             ka.tails = t;
+        }
+        if (!dgrad && choose_wgrad_few(plan, group_m, n, total_m, dev.cus)) {
+            wgrad_few_args(plan, n, dev.n_xcd);
+            plan->total_tiles = ka.total_tiles;
+            plan->detail = "mi355x " + what + " few-row 128x128 " + (f8 ? "bf16-out" : dtype_a == GG_DTYPE_BF16 ? "bf16" : "fp16") +
+                           " grid=" + std::to_string(plan->grid) + " tiles=" + std::to_string(plan->total_tiles);
+            *plan_out = plan;
+            return GG_OK;
         }
         // wgrad's K steps differ per group: no split
         if (dgrad && setup_split_k(plan, dev) != GG_OK) {

@@ -1,5 +1,5 @@
-// Few-row kernel (gg_few.hip): forward and dgrad of groups with few rows, 16-bit and fp8. Host-side
-// interface for the C ABI layer.
+// Few-row kernels: forward and dgrad (gg_few.hip) and wgrad (gg_wfew.hip) of groups with few rows,
+// 16-bit and fp8. Host-side interface for the C ABI layer.
 #pragma once
 
 #include "gg_kernel.h"
@@ -29,5 +29,10 @@ constexpr int kFewInstanceCount = static_cast<int>(sizeof(kFewInstances) / sizeo
 // the instance; the group table in args.groups with total_tiles, or d_total's count, or built in
 // the kernel from d_lens). mn: B is stored contraction-major (dgrad's w).
 hipError_t launch_few_gemm(const KernelArgs &args, int format, bool mn, int instance, int grid, hipStream_t stream);
+
+// The 128 x 128 wgrad kernel (gg_wfew.hip): one workgroup per tile, `grid` of at least
+// args.total_tiles of them (group by group: ceil(m_out / 128) x ceil(n / 128) each).
+constexpr int kWgradFewTile = 128;
+hipError_t launch_wgrad_few(const KernelArgs &args, int format, int grid, hipStream_t stream);
 
 } // namespace gg

@@ -106,12 +106,12 @@ def mean_after_first(ds, key):
 
 
 # The GEMM launch of a plan: the persistent kernel, the small-tile kernel (gg_small.hip) or the
-# few-row kernel (gg_few.hip).
-GEMM_KERNEL = re.compile(r"(?:grouped_gemm_kernel|small_gemm_kernel|few_gemm_kernel)<[^>]*>")
+# few-row kernels (gg_few.hip, gg_wfew.hip).
+GEMM_KERNEL = re.compile(r"(?:grouped_gemm_kernel|small_gemm_kernel|few_gemm_kernel|wgrad_few_kernel)<[^>]*>")
 
 
 def is_gemm(name: str) -> bool:
-    return any(k in name for k in ("grouped_gemm_kernel", "small_gemm_kernel", "few_gemm_kernel"))
+    return any(k in name for k in ("grouped_gemm_kernel", "small_gemm_kernel", "few_gemm_kernel", "wgrad_few_kernel"))
 
 
 def instance(name: str) -> str:

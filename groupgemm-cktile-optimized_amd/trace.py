@@ -40,8 +40,8 @@ def log(msg: str) -> None:
 
 
 # The GEMM launch of a plan: the persistent kernel, the small-tile kernel (gg_small.hip) or the
-# few-row kernel (gg_few.hip).
-GEMM_KERNEL = re.compile(r"(grouped_gemm_kernel|small_gemm_kernel|few_gemm_kernel)<([^>]*)>")
+# few-row kernels (gg_few.hip, gg_wfew.hip).
+GEMM_KERNEL = re.compile(r"(grouped_gemm_kernel|small_gemm_kernel|few_gemm_kernel|wgrad_few_kernel)<([^>]*)>")
 
 
 def mangled_instance(name: str) -> str:
