@@ -23,7 +23,7 @@ from typing import List, Optional, Sequence
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(PKG_DIR, "lib", "libgg_mi355x.so")
 
-GG_OK, GG_ERR_UNSUPPORTED, GG_ERR_INVALID, GG_ERR_HIP = 0, 1, 2, 3
+GG_OK, GG_ERR_UNSUPPORTED, GG_ERR_INVALID, GG_ERR_HIP, GG_ERR_WORKSPACE = 0, 1, 2, 3, 4
 
 # Every symbol include/gg_grouped_gemm.h declares, with its ctypes signature.
 C_API = {
@@ -67,6 +67,16 @@ C_API = {
                                                   ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                                   ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                                   ctypes.c_void_p]),
+    "gg_call": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int64,
+                               ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                               ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
+                               ctypes.POINTER(ctypes.c_size_t), ctypes.c_void_p]),
+    "gg_call_device_lens": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64,
+                                           ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
+                                           ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                           ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p,
+                                           ctypes.c_void_p]),
+    "gg_check_status": (ctypes.c_int, [ctypes.c_void_p]),
     "gg_prepare_dgrad_fp8": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64,
                                             ctypes.c_int64, ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p,
                                             ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
@@ -360,6 +370,53 @@ def _device_sizes(group_m, group_offs, b):
     return True
 
 
+def _one_call(dev, stream: Optional[int]) -> bool:
+    """Whether a torch-level call can take its device memory from torch's allocator (gg_call): work on
+    the current stream of the current device, which that memory belongs to."""
+    import torch
+
+    return stream is None and dev.index == torch.cuda.current_device()
+
+
+def _call_host(op: int, a_dtype: DType, b_dtype: DType, n: int, k: int, group_m: Sequence[int], a, b, out,
+               a_scale=None, b_scale=None) -> None:
+    """One pass over host group sizes on the current stream, waited for (gg_call)."""
+    import torch
+
+    lib, count = load_library(), len(group_m)
+    stream = torch.cuda.current_stream(a.device)
+    gm = (ctypes.c_int64 * max(1, count))(*group_m)
+    need = ctypes.c_size_t(4096 + 16 * count)  # the tables of any plan without partial sums or small tiles
+    sa, sb = (0, 0) if a_scale is None else (a_scale.data_ptr(), b_scale.data_ptr())
+    for _ in range(2):
+        ws = torch.empty(need.value, dtype=torch.uint8, device=a.device)
+        st = lib.gg_call(op, int(a_dtype), int(b_dtype), count, n, k, gm, a.data_ptr(), b.data_ptr(), sa, sb,
+                         out.data_ptr(), ws.data_ptr(), ws.numel(), ctypes.byref(need), stream.cuda_stream)
+        if st != GG_ERR_WORKSPACE:
+            break
+    _check(st)
+    stream.synchronize()
+
+
+def _call_device(op: int, a_dtype: DType, b_dtype: DType, n: int, k: int, group_lens, group_offs, rows: int, a, b, out,
+                 a_scale=None, b_scale=None) -> None:
+    """One pass over device group sizes on the current stream, waited for; raises on sizes that did not
+    fit (gg_call_device_lens)."""
+    import torch
+
+    lib, count = load_library(), group_lens.numel()
+    stream = torch.cuda.current_stream(a.device)
+    ws = torch.empty(16 * (count + 1), dtype=torch.uint8, device=a.device)
+    status = torch.empty(4, dtype=torch.int32, pin_memory=True)
+    sa, sb = (0, 0) if a_scale is None else (a_scale.data_ptr(), b_scale.data_ptr())
+    _check(lib.gg_call_device_lens(op, int(a_dtype), int(b_dtype), count, rows, n, k, group_lens.data_ptr(),
+                                   0 if group_offs is None else group_offs.data_ptr(), a.data_ptr(), b.data_ptr(),
+                                   sa, sb, out.data_ptr(), ws.data_ptr(), ws.numel(), status.data_ptr(),
+                                   stream.cuda_stream))
+    stream.synchronize()
+    _check(lib.gg_check_status(status.data_ptr()))
+
+
 def _run_device_plan(plan: DeviceLensPlan, s: int, dev) -> None:
     import torch
 
@@ -419,6 +476,9 @@ def grouped_gemm_fp8(x, w, group_m: Sequence[int], x_scale, w_scale, out=None, s
         raise ValueError("shape mismatch between x, w, group_m and the scales")
     if out is None:
         out = torch.empty((x.shape[0], n), dtype=torch.bfloat16, device=x.device)
+    if _one_call(x.device, stream):
+        _call_host(OP_FORWARD, kinds[x.dtype], kinds[w.dtype], n, k, group_m, x, w, out, x_scale, w_scale)
+        return out
     s = torch.cuda.current_stream(x.device).cuda_stream if stream is None else stream
     plan = Fp8Plan(kinds[x.dtype], n, k, list(group_m), x.data_ptr(), w.data_ptr(), x_scale.data_ptr(),
                    w_scale.data_ptr(), out.data_ptr(), s)
@@ -555,8 +615,15 @@ def _backward(kind: str, grad_out, other, group_m, out, stream: Optional[int], g
     n, k, shape = _backward_shapes(kind, grad_out, other, group_m, device_sizes)
     if out is None:
         out = torch.empty(shape, dtype=grad_out.dtype, device=grad_out.device)
-    s = torch.cuda.current_stream(grad_out.device).cuda_stream if stream is None else stream
     dt = DType.BF16 if grad_out.dtype == torch.bfloat16 else DType.FP16
+    if _one_call(grad_out.device, stream):
+        op = OP_DGRAD if kind == "dgrad" else OP_WGRAD
+        if device_sizes:
+            _call_device(op, dt, dt, n, k, group_m, group_offs, grad_out.shape[0], grad_out, other, out)
+        else:
+            _call_host(op, dt, dt, n, k, group_m, grad_out, other, out)
+        return out
+    s = torch.cuda.current_stream(grad_out.device).cuda_stream if stream is None else stream
     if device_sizes:
         plan = DeviceLensPlan(OP_DGRAD if kind == "dgrad" else OP_WGRAD, dt, dt, b, grad_out.shape[0], n, k,
                               group_m.data_ptr(), group_offs.data_ptr() if group_offs is not None else 0,
@@ -589,6 +656,14 @@ def _backward_fp8(kind: str, grad_out, other, group_m, grad_scale, other_scale, 
     n, k, shape = _backward_shapes(kind, grad_out, other, group_m, device_sizes)
     if out is None:
         out = torch.empty(shape, dtype=torch.bfloat16, device=grad_out.device)
+    if _one_call(grad_out.device, stream):
+        op, ka, kb = OP_DGRAD if kind == "dgrad" else OP_WGRAD, kinds[grad_out.dtype], kinds[other.dtype]
+        if device_sizes:
+            _call_device(op, ka, kb, n, k, group_m, group_offs, grad_out.shape[0], grad_out, other, out, grad_scale,
+                         other_scale)
+        else:
+            _call_host(op, ka, kb, n, k, group_m, grad_out, other, out, grad_scale, other_scale)
+        return out
     s = torch.cuda.current_stream(grad_out.device).cuda_stream if stream is None else stream
     if device_sizes:
         plan = DeviceLensPlan(OP_DGRAD if kind == "dgrad" else OP_WGRAD, kinds[grad_out.dtype], kinds[other.dtype],
@@ -679,8 +754,14 @@ def grouped_gemm(x, w, group_m, out=None, stream: Optional[int] = None, group_of
         raise ValueError("shape mismatch between x, w and group_m")
     if out is None:
         out = torch.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
-    s = torch.cuda.current_stream(x.device).cuda_stream if stream is None else stream
     dt = DType.BF16 if x.dtype == torch.bfloat16 else DType.FP16
+    if _one_call(x.device, stream):
+        if device_sizes:
+            _call_device(OP_FORWARD, dt, dt, n, k, group_m, group_offs, x.shape[0], x, w, out)
+        else:
+            _call_host(OP_FORWARD, dt, dt, n, k, group_m, x, w, out)
+        return out
+    s = torch.cuda.current_stream(x.device).cuda_stream if stream is None else stream
     be = Mi355xBackend()
     if device_sizes:
         why = be.prepare_device_lens(dt, b, x.shape[0], n, k, group_m.data_ptr(),

@@ -11,6 +11,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <mutex>
 #include <new>
 #include <string>
@@ -32,6 +33,14 @@ struct gg_plan {
     const void         *x           = nullptr;
     const void         *w           = nullptr;
     void               *out         = nullptr;
+    // What the launch reads on the device, filled on the host by the plan builders; bind_plan places
+    // it (and ws_bytes of workspace) in device memory, `mem` if the plan owns that.
+    std::vector<gg::GroupEntry> table;
+    std::vector<gg::TileDesc>   desc;
+    std::vector<gg::SmallTile>  small_list;
+    size_t                      ws_bytes = 0;
+    void                       *mem      = nullptr;
+    bool                        one_call = false; // gg_call: no descriptors, no detail text
     gg::GroupEntry     *d_groups    = nullptr;
     gg::KernelArgs      args{};
     std::string         detail;
@@ -41,13 +50,10 @@ struct gg_plan {
     const int64_t      *d_offs      = nullptr;
     gg::TableHeader    *d_header    = nullptr; // follows the table in the d_groups allocation
     bool                in_kernel_table = false; // the GEMM builds the table (no table launch)
-    float              *d_ws        = nullptr; // split-K / tail-split partial sums (args.ws)
-    gg::TileDesc       *d_desc      = nullptr; // tile descriptors (args.desc)
     int64_t             in_rows     = 0;       // device-size plans: rows of the inputs
     // Small-tile plans (use_small_tiles): the launch of gg_small.hip instead of the persistent one.
     bool                small       = false;
     gg::SmallArgs       sargs{};
-    gg::SmallTile      *d_small     = nullptr; // [sargs.tiles]
     int                 few         = -1;      // few-row plans: the instance of gg_few.hip, -1: none
     bool                wgrad_few   = false;   // wgrad plans: the kernel of gg_wfew.hip
 };
@@ -204,23 +210,18 @@ int choose_splits(int tiles, int k_tiles, int cus) {
 // tile each (1 x 2048 x 7168: 224 tiles of 256 x 256 on 256 CUs, 256 tiles of 256 x 224). The
 // group table is rebuilt for the narrow tile count. GG_NARROW=0 in the environment turns this
 // off.
-int use_narrow_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, hipStream_t s) {
+void use_narrow_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev) {
     gg::KernelArgs &a   = plan->args;
     const char     *env = std::getenv("GG_NARROW");
     if ((env != nullptr && *env != '\0' && std::atoi(env) == 0) || a.splits > 1 || a.tile_m != gg::kTileM ||
         plan->total_tiles >= dev.cus)
-        return GG_OK;
+        return;
     const int64_t               n_tiles = gg::cdiv(plan->n, gg::kNarrowTileN);
     std::vector<gg::GroupEntry> table(static_cast<size_t>(plan->group_num));
     const int64_t tiles = gg::build_group_table(group_m, plan->group_num, n_tiles, table.data());
     if (tiles <= plan->total_tiles || tiles > dev.cus)
-        return GG_OK;
-    hipError_t e = hipMemcpyAsync(plan->d_groups, table.data(), table.size() * sizeof(gg::GroupEntry),
-                                  hipMemcpyHostToDevice, s);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(s);
-    if (e != hipSuccess)
-        return hip_fail(e, "narrow group table upload");
+        return;
+    plan->table       = std::move(table);
     plan->total_tiles = static_cast<int>(tiles);
     plan->grid        = plan->total_tiles;
     a.total_tiles     = plan->total_tiles;
@@ -228,7 +229,6 @@ int use_narrow_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, h
     a.tile_n          = gg::kNarrowTileN;
     const int n_xcd   = dev.n_xcd;
     a.n_xcd           = plan->grid % n_xcd == 0 ? n_xcd : 1;
-    return GG_OK;
 }
 
 // Modelled time, in full 256 x 256 tile steps, of the busiest workgroup when tiles of tile_m rows
@@ -270,7 +270,7 @@ double busiest_workgroup(const int64_t *group_m, int group_num, int64_t n_tiles,
 // 176 rows per group; 4.71 -> 4.36 tile steps). The group table is rebuilt for the tile rows.
 // GG_SHORT=0 in the environment turns this off, GG_SHORT=1 takes short tiles whenever the tile
 // counts allow.
-int use_short_tiles(gg_plan *plan, const int64_t *group_m, hipStream_t s) {
+int use_short_tiles(gg_plan *plan, const int64_t *group_m) {
     gg::KernelArgs &a   = plan->args;
     const char     *env = std::getenv("GG_SHORT");
     const int       opt = env != nullptr && *env != '\0' ? std::atoi(env) : -1;
@@ -291,12 +291,7 @@ int use_short_tiles(gg_plan *plan, const int64_t *group_m, hipStream_t s) {
     const int64_t tiles = gg::build_group_table(group_m, plan->group_num, a.n_tiles, table.data(), 0, rows);
     if (tiles != plan->total_tiles)
         return fail(GG_ERR_INVALID, "short tiles changed the tile count");
-    hipError_t e = hipMemcpyAsync(plan->d_groups, table.data(), table.size() * sizeof(gg::GroupEntry),
-                                  hipMemcpyHostToDevice, s);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(s);
-    if (e != hipSuccess)
-        return hip_fail(e, "short group table upload");
+    plan->table = std::move(table);
     a.tile_m = rows;
     return GG_OK;
 }
@@ -312,18 +307,18 @@ int use_short_tiles(gg_plan *plan, const int64_t *group_m, hipStream_t s) {
 // plan allows them.
 constexpr double kWideTileCost = 1.10;
 
-int use_short_wide_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, hipStream_t s) {
+void use_short_wide_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev) {
     gg::KernelArgs &a   = plan->args;
     const char     *env = std::getenv("GG_WIDE");
     const int       opt = env != nullptr && *env != '\0' ? std::atoi(env) : -1;
     if (opt == 0 || plan->mode != gg::make_mode(gg::kFwd, gg::kIn16) || a.tile_m == gg::kTileM ||
         a.tile_n != gg::kTileN || a.splits > 1 || a.d_total != nullptr || a.d_lens != nullptr)
-        return GG_OK;
+        return;
     const int64_t n_tiles = gg::cdiv(plan->n, gg::kShortWideTileN);
     std::vector<gg::GroupEntry> table(static_cast<size_t>(plan->group_num));
     const int64_t tiles = gg::build_group_table(group_m, plan->group_num, n_tiles, table.data(), 0, a.tile_m);
     if (tiles <= 0 || tiles > INT32_MAX)
-        return GG_OK;
+        return;
     const int grid  = static_cast<int>(std::min<int64_t>(dev.cus, tiles));
     const int n_xcd = grid % dev.n_xcd == 0 ? dev.n_xcd : 1;
     gg::KernelArgs w = a;
@@ -332,41 +327,30 @@ int use_short_wide_tiles(gg_plan *plan, const int64_t *group_m, const Device &de
     w.tile_n         = gg::kShortWideTileN;
     w.n_xcd          = n_xcd;
     if (!gg::uses_cross_tile(w, grid, plan->mode))
-        return GG_OK;
+        return;
     if (opt != 1) {
         const double short_ = busiest_workgroup(group_m, plan->group_num, a.n_tiles, a.tile_m, plan->total_tiles,
                                                 plan->grid, a.n_xcd, a.band);
         const double wide   = kWideTileCost * busiest_workgroup(group_m, plan->group_num, n_tiles, a.tile_m,
                                                                 w.total_tiles, grid, n_xcd, a.band);
         if (wide > 0.95 * short_)
-            return GG_OK;
+            return;
     }
-    hipError_t e = hipMemcpyAsync(plan->d_groups, table.data(), table.size() * sizeof(gg::GroupEntry),
-                                  hipMemcpyHostToDevice, s);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(s);
-    if (e != hipSuccess)
-        return hip_fail(e, "short-wide group table upload");
+    plan->table       = std::move(table);
     plan->total_tiles = w.total_tiles;
     plan->grid        = grid;
     a                 = w;
-    return GG_OK;
 }
 
-// Picks the plan's split count (plan->args filled, k_tiles set) and allocates the partial sums.
-int setup_split_k(gg_plan *plan, const Device &dev) {
+// Picks the plan's split count (plan->args filled, k_tiles set) and the size of its partial sums.
+void setup_split_k(gg_plan *plan, const Device &dev) {
     gg::KernelArgs &a  = plan->args;
     const int       sp = choose_splits(plan->total_tiles, a.k_tiles, dev.cus);
     if (sp <= 1)
-        return GG_OK;
-    const size_t bytes = size_t(sp) * size_t(plan->total_tiles) * 262144;
-    const hipError_t e = hipMalloc(&plan->d_ws, bytes);
-    if (e != hipSuccess)
-        return hip_fail(e, "split-K workspace allocation");
-    a.splits    = sp;
-    a.ws        = plan->d_ws;
-    plan->grid  = static_cast<int>(std::min<int64_t>(dev.cus, int64_t(sp) * plan->total_tiles));
-    return GG_OK;
+        return;
+    plan->ws_bytes = size_t(sp) * size_t(plan->total_tiles) * 262144;
+    a.splits       = sp;
+    plan->grid     = static_cast<int>(std::min<int64_t>(dev.cus, int64_t(sp) * plan->total_tiles));
 }
 
 // Tail split for cross-tile 16-bit forward plans (host-size tables): when the last round holds
@@ -387,34 +371,30 @@ constexpr double kTailStoreUs  = 6.0;
 constexpr double kTailLaunchUs = 5.0;
 constexpr double kTailTileUs   = 0.15;
 
-int setup_tail_split(gg_plan *plan) {
+void setup_tail_split(gg_plan *plan) {
     gg::KernelArgs &a = plan->args;
     a.tail_splits     = 1;
     if (plan->mode != gg::make_mode(gg::kFwd, gg::kIn16) || a.splits > 1 || a.d_total != nullptr ||
         a.d_lens != nullptr || a.tile_n != gg::kTileN || !gg::uses_cross_tile(a, plan->grid, plan->mode))
-        return GG_OK;
+        return;
     const int grid = plan->grid, tiles = plan->total_tiles;
     const int full = tiles / grid * grid, rem = tiles - full;
     if (full == 0 || rem == 0 || 2 * rem > grid)
-        return GG_OK;
+        return;
     int forced = -1;
     if (const char *env = std::getenv("GG_TAIL_SPLIT"); env != nullptr && *env != '\0')
         forced = std::atoi(env);
     if (forced == 0 || forced == 1)
-        return GG_OK;
+        return;
     constexpr int sp = 2;
     if (a.k_tiles / sp < (forced > 1 ? gg::kCrossMinStepsHost : kMinTailSteps))
-        return GG_OK;
+        return;
     const double saved_us = (a.k_tiles - gg::cdiv(a.k_tiles, sp)) * kStepUs;
     const double cost_us  = kTailStoreUs + kTailLaunchUs + rem * kTailTileUs;
     if (forced < 0 && saved_us < 1.1 * cost_us)
-        return GG_OK;
-    const hipError_t e = hipMalloc(&plan->d_ws, size_t(rem) * size_t(sp) * 262144);
-    if (e != hipSuccess)
-        return hip_fail(e, "tail-split workspace");
-    a.tail_splits = sp;
-    a.ws          = plan->d_ws;
-    return GG_OK;
+        return;
+    plan->ws_bytes = size_t(rem) * size_t(sp) * 262144;
+    a.tail_splits  = sp;
 }
 
 // Small tiles (128 x 128, one per workgroup, gg_small.hip) for 16-bit forward plans of host-size
@@ -451,13 +431,13 @@ bool small_tiles_win(int64_t units, int per, int tiles, int splits, int k_tiles,
     return kSmallFixedUs + double(per) * step <= kSmallGain * big;
 }
 
-int use_small_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, hipStream_t s) {
+void use_small_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev) {
     const char *env = std::getenv("GG_SMALL");
     const int   opt = env != nullptr && *env != '\0' ? std::atoi(env) : -1;
     const int   cus = dev.cus;
     const gg::KernelArgs &a = plan->args;
     if (opt == 0 || plan->group_num > 32767 || (opt != 1 && (2 * plan->total_tiles > cus || a.tail_splits > 1)))
-        return GG_OK;
+        return;
     const int64_t              nt = gg::cdiv(plan->n, gg::kSmallTile);
     std::vector<gg::SmallTile> list;
     int64_t                    row = 0;
@@ -473,7 +453,7 @@ int use_small_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, hi
     const int64_t tiles   = static_cast<int64_t>(list.size());
     const int     k_steps = static_cast<int>(gg::cdiv(plan->k, gg::kSmallK));
     if (tiles == 0 || tiles > 65536)
-        return GG_OK;
+        return;
     // Workgroup i runs on XCD i % n_xcd: deal the list (N-tile by N-tile, M-tiles inside) to the
     // XCDs in contiguous runs (xcd_remap), so that the workgroups of one XCD share a few x and w
     // panels in its L2 instead of every XCD reading every w panel.
@@ -495,30 +475,16 @@ int use_small_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, hi
     // a 4-step ring while every workgroup has a CU of its own, else a 2-step ring, two per CU
     const int stages = tiles * sp <= cus ? gg::kSmallStagesOne : gg::kSmallStagesTwo;
     if (opt != 1 && !small_tiles_win(tiles * sp, per, plan->total_tiles, a.splits, a.k_tiles, cus))
-        return GG_OK;
-    // the persistent plan's workspace and descriptors are not used by this launch
-    if (plan->d_ws != nullptr)
-        (void)hipFree(plan->d_ws);
-    if (plan->d_desc != nullptr)
-        (void)hipFree(plan->d_desc);
-    plan->d_ws   = nullptr;
-    plan->d_desc = nullptr;
-    const size_t bytes = list.size() * sizeof(gg::SmallTile);
-    hipError_t   e     = hipMalloc(&plan->d_small, bytes);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(plan->d_small, list.data(), bytes, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(s);
-    if (e == hipSuccess && sp > 1)
-        e = hipMalloc(&plan->d_ws, size_t(sp) * size_t(tiles) * gg::kSmallTile * gg::kSmallTile * sizeof(float));
-    if (e != hipSuccess)
-        return hip_fail(e, "small-tile plan");
+        return;
+    // the persistent plan's table, workspace and descriptors are not used by this launch
+    plan->table.clear();
+    plan->desc.clear();
+    plan->ws_bytes   = sp > 1 ? size_t(sp) * size_t(tiles) * gg::kSmallTile * gg::kSmallTile * sizeof(float) : 0;
+    plan->small_list = std::move(list);
     gg::SmallArgs &sa    = plan->sargs;
     sa.x                 = plan->x;
     sa.w                 = plan->w;
     sa.out               = plan->out;
-    sa.tile_list         = plan->d_small;
-    sa.ws                = plan->d_ws;
     sa.tiles             = static_cast<int>(tiles);
     sa.n                 = static_cast<int>(plan->n);
     sa.k                 = static_cast<int>(plan->k);
@@ -529,19 +495,60 @@ int use_small_tiles(gg_plan *plan, const int64_t *group_m, const Device &dev, hi
     plan->small          = true;
     plan->total_tiles    = static_cast<int>(tiles);
     plan->grid           = static_cast<int>(tiles) * sp;
-    return GG_OK;
 }
 
 void free_plan(gg_plan *plan) {
-    if (plan->d_small != nullptr)
-        (void)hipFree(plan->d_small);
-    if (plan->d_groups != nullptr)
-        (void)hipFree(plan->d_groups);
-    if (plan->d_ws != nullptr)
-        (void)hipFree(plan->d_ws);
-    if (plan->d_desc != nullptr)
-        (void)hipFree(plan->d_desc);
+    if (plan->mem != nullptr)
+        (void)hipFree(plan->mem);
     delete plan;
+}
+
+// ---------------------------------------------------------------------------------------
+// Placing a host-size plan's tables and workspace in device memory: one block, its parts at
+// multiples of 256 bytes, the workspace last (nothing is uploaded into it).
+// ---------------------------------------------------------------------------------------
+size_t block(size_t bytes) { return (bytes + 255) / 256 * 256; }
+size_t upload_bytes(const gg_plan *p) {
+    return block(p->table.size() * sizeof(gg::GroupEntry)) + block(p->desc.size() * sizeof(gg::TileDesc)) +
+           block(p->small_list.size() * sizeof(gg::SmallTile));
+}
+size_t plan_bytes(const gg_plan *p) { return upload_bytes(p) + p->ws_bytes; }
+
+// Points the plan's arguments into `mem` (plan_bytes of device memory) and writes what belongs there
+// to `image` (upload_bytes).
+void bind_plan(gg_plan *p, void *mem, std::vector<char> *image) {
+    image->assign(upload_bytes(p), 0);
+    size_t     at    = 0;
+    const auto place = [&](const auto &v) {
+        char *dst = v.empty() ? nullptr : static_cast<char *>(mem) + at;
+        if (!v.empty())
+            std::memcpy(image->data() + at, v.data(), v.size() * sizeof(v[0]));
+        at += block(v.size() * sizeof(v[0]));
+        return dst;
+    };
+    p->d_groups        = reinterpret_cast<gg::GroupEntry *>(place(p->table));
+    p->args.groups     = p->d_groups;
+    p->args.desc       = reinterpret_cast<const int *>(place(p->desc));
+    p->sargs.tile_list = reinterpret_cast<gg::SmallTile *>(place(p->small_list));
+    p->args.ws         = p->ws_bytes > 0 ? reinterpret_cast<float *>(static_cast<char *>(mem) + at) : nullptr;
+    p->sargs.ws        = p->args.ws;
+}
+
+// Device memory of a plan that owns it, uploaded on `s` and waited for.
+int allocate_plan(gg_plan *p, hipStream_t s) {
+    if (plan_bytes(p) == 0)
+        return GG_OK;
+    hipError_t e = hipMalloc(&p->mem, plan_bytes(p));
+    if (e != hipSuccess) {
+        p->mem = nullptr;
+        return hip_fail(e, "plan memory allocation");
+    }
+    std::vector<char> image;
+    bind_plan(p, p->mem, &image);
+    e = hipMemcpyAsync(p->mem, image.data(), image.size(), hipMemcpyHostToDevice, s);
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(s);
+    return e == hipSuccess ? GG_OK : hip_fail(e, "plan table upload");
 }
 
 // Few-row tiles (gg_few.hip) for forward and dgrad plans, 16-bit and fp8, host- and device-size,
@@ -736,7 +743,7 @@ void wgrad_few_args(gg_plan *plan, int64_t m_out, int n_xcd) {
 // Turns a host-size forward or dgrad plan (its problem set) into a few-row plan where
 // choose_few_rows takes one: the group table of the instance's tiles and the launch.
 int use_few_rows(gg_plan *plan, const int64_t *group_m, const float *x_scale, const float *w_scale,
-                 const std::string &what, hipStream_t s) {
+                 const std::string &what) {
     Device dev;
     if (current_device(&dev) != GG_OK)
         return GG_ERR_HIP;
@@ -748,14 +755,7 @@ int use_few_rows(gg_plan *plan, const int64_t *group_m, const float *x_scale, co
     const int64_t tiles = gg::build_group_table(group_m, plan->group_num, gg::cdiv(plan->n, f.tile_n), table.data(), 0, f.tile_m);
     if (tiles <= 0)
         return GG_OK;
-    const size_t bytes = table.size() * sizeof(gg::GroupEntry);
-    hipError_t   e     = hipMalloc(&plan->d_groups, bytes);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(plan->d_groups, table.data(), bytes, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(s);
-    if (e != hipSuccess)
-        return hip_fail(e, "few-row group table");
+    plan->table       = std::move(table);
     plan->few         = few;
     plan->total_tiles = static_cast<int>(tiles);
     plan->grid        = 0;
@@ -766,7 +766,8 @@ int use_few_rows(gg_plan *plan, const int64_t *group_m, const float *x_scale, co
     plan->args.total_tiles = plan->total_tiles;
     plan->args.x_scale     = x_scale;
     plan->args.w_scale     = w_scale;
-    plan->detail           = few_detail(plan, what);
+    if (!plan->one_call)
+        plan->detail = few_detail(plan, what);
     return GG_OK;
 }
 
@@ -777,10 +778,10 @@ int use_few_rows(gg_plan *plan, const int64_t *group_m, const float *x_scale, co
 // (the kernel walks the table itself) with split-K, a tail split, more than kMaxDescPerWg tiles
 // per workgroup or rows past 2^31 (output rows, and for wgrad the input tokens whose offsets its
 // descriptors hold). GG_TILE_DESC=0 in the environment turns them off.
-int setup_tile_desc(gg_plan *plan, const int64_t *group_m, hipStream_t s) {
+int setup_tile_desc(gg_plan *plan, const int64_t *group_m) {
     gg::KernelArgs &a   = plan->args;
     const char     *env = std::getenv("GG_TILE_DESC");
-    if ((env != nullptr && env[0] == '0') || a.splits > 1 || a.tail_splits > 1 || plan->grid <= 0 ||
+    if ((env != nullptr && env[0] == '0') || plan->one_call || a.splits > 1 || a.tail_splits > 1 || plan->grid <= 0 ||
         !gg::desc_rows_fit(group_m, plan->group_num, plan->total_m))
         return GG_OK;
     const int per_wg = static_cast<int>(gg::cdiv(plan->total_tiles, plan->grid));
@@ -816,15 +817,7 @@ int setup_tile_desc(gg_plan *plan, const int64_t *group_m, hipStream_t s) {
             desc[static_cast<size_t>(wg) * per_wg + i] = gg::TileDesc{static_cast<int32_t>(r0), g, (tn << 9) | mv, 0};
         }
     }
-    const size_t bytes = desc.size() * sizeof(gg::TileDesc);
-    hipError_t   e     = hipMalloc(&plan->d_desc, bytes);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(plan->d_desc, desc.data(), bytes, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(s);
-    if (e != hipSuccess)
-        return hip_fail(e, "tile descriptor upload");
-    a.desc        = reinterpret_cast<const int *>(plan->d_desc);
+    plan->desc    = std::move(desc);
     a.desc_per_wg = per_wg;
     return GG_OK;
 }
@@ -875,10 +868,14 @@ int noalloc_scratch(void **out) {
 }
 
 // Validates a device-size problem (the rules of gg_prepare_device_lens_op) and fills *plan.
-// noalloc = false: the table and header are one hipMalloc owned by the plan (free_plan releases
-// it, also on failure). noalloc = true: they are the current device's scratch array, and nothing
-// is allocated (no detail text either). A plan without a launch keeps d_groups null.
-int plan_device_lens(gg_plan *plan, bool noalloc, int op, int a_dtype, int b_dtype, int group_num,
+// The group table and its header live in a hipMalloc'd block that the plan owns (kOwned: free_plan
+// releases it, also on failure), in the current device's scratch array (kScratch) or in `given`
+// (kGiven: device_table_bytes of device memory); only kOwned plans have a detail text. A plan without
+// a launch keeps d_groups null.
+enum TableMemory { kOwned, kScratch, kGiven };
+size_t device_table_bytes(int group_num) { return size_t(group_num) * sizeof(gg::GroupEntry) + sizeof(gg::TableHeader); }
+
+int plan_device_lens(gg_plan *plan, TableMemory memory, void *given, int op, int a_dtype, int b_dtype, int group_num,
                      int64_t total_m, int64_t n, int64_t k, const int64_t *group_lens, const int64_t *group_offs,
                      const void *a, const void *b, const float *a_scale, const float *b_scale, void *out) {
     if (op != GG_OP_FORWARD && op != GG_OP_DGRAD && op != GG_OP_WGRAD)
@@ -953,6 +950,7 @@ int plan_device_lens(gg_plan *plan, bool noalloc, int op, int a_dtype, int b_dty
     plan->device_lens = true;
     plan->d_lens      = group_lens;
     plan->d_offs      = group_offs;
+    const bool  noalloc = memory != kOwned;
     std::string what;
     if (!noalloc)
         what = std::string(op == GG_OP_FORWARD ? "" : op == GG_OP_DGRAD ? "dgrad " : "wgrad ") +
@@ -978,21 +976,23 @@ int plan_device_lens(gg_plan *plan, bool noalloc, int op, int a_dtype, int b_dty
     if (const int st = current_device(&dev); st != GG_OK)
         return st;
     const int cus = dev.cus, n_xcd = dev.n_xcd;
-    if (noalloc) {
+    if (memory == kScratch) {
         void *mem = nullptr;
         if (const int st = noalloc_scratch(&mem); st != GG_OK)
             return st;
         plan->d_groups = static_cast<gg::GroupEntry *>(mem);
         plan->d_header = reinterpret_cast<gg::TableHeader *>(static_cast<char *>(mem) + kNoAllocTableBytes);
     } else {
-        // Table + header in one allocation; the header is written by every run.
-        const hipError_t e = hipMalloc(&plan->d_groups, table_bytes + sizeof(gg::TableHeader));
-        if (e != hipSuccess) {
-            plan->d_groups = nullptr;
-            return hip_fail(e, "group table allocation");
+        if (memory == kOwned) { // one allocation; the header is written by every run
+            const hipError_t e = hipMalloc(&plan->mem, device_table_bytes(group_num));
+            if (e != hipSuccess) {
+                plan->mem = nullptr;
+                return hip_fail(e, "group table allocation");
+            }
+            given = plan->mem;
         }
-        plan->d_header = reinterpret_cast<gg::TableHeader *>(reinterpret_cast<char *>(plan->d_groups) +
-                                                             table_bytes);
+        plan->d_groups = static_cast<gg::GroupEntry *>(given);
+        plan->d_header = reinterpret_cast<gg::TableHeader *>(static_cast<char *>(given) + table_bytes);
     }
     fill_args(plan, 1);
     gg::KernelArgs &ka = plan->args;
@@ -1131,15 +1131,11 @@ int run_plan(const gg_plan *plan, void *stream, bool zero_kernel) {
 
 extern "C" {
 
-int gg_prepare(int dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
-               const void *x, const void *w, void *out, void *stream, gg_plan **plan_out) {
-    g_last_error.clear();
-    if (plan_out == nullptr)
-        return fail(GG_ERR_INVALID, "plan_out is null");
-    *plan_out = nullptr;
+// Validates a host-size forward problem and fills *plan (nothing on the device).
+static int plan_forward(gg_plan *plan, int dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
+                        const void *x, const void *w, void *out) {
     if (group_num > 0 && group_m == nullptr)
         return fail(GG_ERR_INVALID, "group_m is null");
-
     int64_t total_m = 0;
     for (int g = 0; g < group_num; ++g) {
         if (group_m[g] < 0)
@@ -1151,9 +1147,6 @@ int gg_prepare(int dtype, int group_num, int64_t n, int64_t k, const int64_t *gr
     if (st != GG_OK)
         return st;
 
-    auto *plan = new (std::nothrow) gg_plan;
-    if (plan == nullptr)
-        return fail(GG_ERR_INVALID, "out of host memory");
     plan->dtype     = dtype;
     plan->group_num = group_num;
     plan->n         = n;
@@ -1166,98 +1159,82 @@ int gg_prepare(int dtype, int group_num, int64_t n, int64_t k, const int64_t *gr
     // Group table: row offset, rows and first tile of every group (empty groups own no
     // tiles; the kernel steps over them while scanning forward).
     const int64_t n_tiles = gg::cdiv(n, gg::kTileN);
-    std::vector<gg::GroupEntry> table(static_cast<size_t>(group_num));
-    const int64_t tiles = gg::build_group_table(group_m, group_num, n_tiles, table.data());
-    if (tiles < 0) {
-        delete plan;
+    plan->table.resize(static_cast<size_t>(group_num));
+    const int64_t tiles = gg::build_group_table(group_m, group_num, n_tiles, plan->table.data());
+    if (tiles < 0)
         return fail(GG_ERR_UNSUPPORTED, "too many rows or tiles for 32-bit tile indices");
-    }
     plan->total_tiles = has_output && k > 0 ? static_cast<int>(tiles) : 0;
-
-    const hipStream_t s = static_cast<hipStream_t>(stream);
-    if (plan->total_tiles > 0) {
-        if (use_few_rows(plan, group_m, nullptr, nullptr, dtype == GG_DTYPE_BF16 ? "bf16" : "fp16", s) != GG_OK) {
-            free_plan(plan);
-            return GG_ERR_HIP;
-        }
-        if (plan->few >= 0) {
-            *plan_out = plan;
-            return GG_OK;
-        }
+    if (plan->total_tiles == 0) {
+        plan->table.clear();
+        plan->detail = "mi355x: no launch (" + std::string(has_output ? "K = 0, zero fill" : "empty output") + ")";
+        return GG_OK;
     }
-    if (plan->total_tiles > 0) {
-        Device dev;
-        if (current_device(&dev) != GG_OK) {
-            delete plan;
-            return GG_ERR_HIP;
-        }
-        const size_t bytes = table.size() * sizeof(gg::GroupEntry);
-        hipError_t   e     = hipMalloc(&plan->d_groups, bytes);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(plan->d_groups, table.data(), bytes, hipMemcpyHostToDevice, s);
-        if (e == hipSuccess)
-            e = hipStreamSynchronize(s);
-        if (e != hipSuccess) {
-            if (plan->d_groups != nullptr)
-                (void)hipFree(plan->d_groups);
-            delete plan;
-            return hip_fail(e, "group table upload");
-        }
-        // Persistent grid: one workgroup per CU (160 KB of LDS each), never more than tiles.
-        plan->grid = std::min(dev.cus, plan->total_tiles);
-        fill_args(plan, dev.n_xcd);
-        gg::KernelArgs &a = plan->args;
-        a.total_tiles     = plan->total_tiles;
-        a.d_total         = nullptr;
-        a.tails           = k % gg::kTileK != 0; // K-major operands: only a partial K step
-        if (setup_split_k(plan, dev) != GG_OK) {
-            free_plan(plan);
-            return GG_ERR_HIP;
-        }
-        if (const int st2 = use_short_tiles(plan, group_m, s); st2 != GG_OK) {
-            free_plan(plan);
-            return st2;
-        }
-        if (use_short_wide_tiles(plan, group_m, dev, s) != GG_OK) {
-            free_plan(plan);
-            return GG_ERR_HIP;
-        }
-        if (use_narrow_tiles(plan, group_m, dev, s) != GG_OK) {
-            free_plan(plan);
-            return GG_ERR_HIP;
-        }
-        if (setup_tail_split(plan) != GG_OK) {
-            free_plan(plan);
-            return GG_ERR_HIP;
-        }
-        if (const int st3 = setup_tile_desc(plan, group_m, s); st3 != GG_OK) {
-            free_plan(plan);
-            return st3;
-        }
-        if (const int st4 = use_small_tiles(plan, group_m, dev, s); st4 != GG_OK) {
-            free_plan(plan);
-            return st4;
-        }
-        const std::string dt = dtype == GG_DTYPE_BF16 ? "bf16" : "fp16";
-        if (plan->small)
-            plan->detail = "mi355x small 128x128x64 " + dt + " grid=" + std::to_string(plan->grid) +
-                           " tiles=" + std::to_string(plan->total_tiles) +
-                           (plan->sargs.stages == gg::kSmallStagesTwo ? " two-per-cu" : "") +
-                           (plan->sargs.splits > 1 ? " split-k=" + std::to_string(plan->sargs.splits) : "");
-        else
-            plan->detail = "mi355x persistent " + std::to_string(a.tile_m) + "x" + std::to_string(a.tile_n) +
-                           "x64 " + dt + " grid=" + std::to_string(plan->grid) +
-                           " tiles=" + std::to_string(plan->total_tiles) + " xcd=" + std::to_string(a.n_xcd) +
-                           (gg::uses_cross_tile(a, plan->grid) ? " cross-tile" : " per-tile") +
-                           (a.band != gg::kBand ? " band=" + std::to_string(a.band) : "") +
-                           (a.splits > 1 ? " split-k=" + std::to_string(a.splits) : "") +
-                           (a.tail_splits > 1 ? " tail-split=" + std::to_string(a.tail_splits) : "");
-    } else {
-        plan->detail = "mi355x: no launch (" +
-                       std::string(has_output ? "K = 0, zero fill" : "empty output") + ")";
+    if (const int st2 = use_few_rows(plan, group_m, nullptr, nullptr, dtype == GG_DTYPE_BF16 ? "bf16" : "fp16");
+        st2 != GG_OK || plan->few >= 0)
+        return st2;
+    Device dev;
+    if (current_device(&dev) != GG_OK)
+        return GG_ERR_HIP;
+    // Persistent grid: one workgroup per CU (160 KB of LDS each), never more than tiles.
+    plan->grid = std::min(dev.cus, plan->total_tiles);
+    fill_args(plan, dev.n_xcd);
+    gg::KernelArgs &a = plan->args;
+    a.total_tiles     = plan->total_tiles;
+    a.d_total         = nullptr;
+    a.tails           = k % gg::kTileK != 0; // K-major operands: only a partial K step
+    setup_split_k(plan, dev);
+    if (const int st2 = use_short_tiles(plan, group_m); st2 != GG_OK)
+        return st2;
+    use_short_wide_tiles(plan, group_m, dev);
+    use_narrow_tiles(plan, group_m, dev);
+    setup_tail_split(plan);
+    if (const int st2 = setup_tile_desc(plan, group_m); st2 != GG_OK)
+        return st2;
+    use_small_tiles(plan, group_m, dev);
+    if (plan->one_call)
+        return GG_OK;
+    const std::string dt = dtype == GG_DTYPE_BF16 ? "bf16" : "fp16";
+    if (plan->small)
+        plan->detail = "mi355x small 128x128x64 " + dt + " grid=" + std::to_string(plan->grid) +
+                       " tiles=" + std::to_string(plan->total_tiles) +
+                       (plan->sargs.stages == gg::kSmallStagesTwo ? " two-per-cu" : "") +
+                       (plan->sargs.splits > 1 ? " split-k=" + std::to_string(plan->sargs.splits) : "");
+    else
+        plan->detail = "mi355x persistent " + std::to_string(a.tile_m) + "x" + std::to_string(a.tile_n) +
+                       "x64 " + dt + " grid=" + std::to_string(plan->grid) +
+                       " tiles=" + std::to_string(plan->total_tiles) + " xcd=" + std::to_string(a.n_xcd) +
+                       (gg::uses_cross_tile(a, plan->grid) ? " cross-tile" : " per-tile") +
+                       (a.band != gg::kBand ? " band=" + std::to_string(a.band) : "") +
+                       (a.splits > 1 ? " split-k=" + std::to_string(a.splits) : "") +
+                       (a.tail_splits > 1 ? " tail-split=" + std::to_string(a.tail_splits) : "");
+    return GG_OK;
+}
+
+// A prepare entry point: a new plan, filled by `fill`, its device memory allocated and uploaded.
+extern "C++" {
+template <typename F> static int new_plan(gg_plan **plan_out, void *stream, F fill) {
+    g_last_error.clear();
+    if (plan_out == nullptr)
+        return fail(GG_ERR_INVALID, "plan_out is null");
+    *plan_out  = nullptr;
+    auto *plan = new (std::nothrow) gg_plan;
+    if (plan == nullptr)
+        return fail(GG_ERR_INVALID, "out of host memory");
+    int st = fill(plan);
+    if (st == GG_OK)
+        st = allocate_plan(plan, static_cast<hipStream_t>(stream));
+    if (st != GG_OK) {
+        free_plan(plan);
+        return st;
     }
     *plan_out = plan;
     return GG_OK;
+}
+}
+
+int gg_prepare(int dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
+               const void *x, const void *w, void *out, void *stream, gg_plan **plan_out) {
+    return new_plan(plan_out, stream, [&](gg_plan *plan) { return plan_forward(plan, dtype, group_num, n, k, group_m, x, w, out); });
 }
 
 // Backward plans in kernel terms (see KernelArgs): out (rows x N) = A B^T per group with the
@@ -1267,13 +1244,9 @@ int gg_prepare(int dtype, int group_num, int64_t n, int64_t k, const int64_t *gr
 // dtype_a / dtype_b: formats of grad_out and of the other operand. 16-bit: both the same, no
 // scales. fp8: e4m3 x e4m3, e5m2 x e5m2 or e5m2 gradient x e4m3, bf16 out scaled by a_scale[0] *
 // b_scale[g].
-static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num, int64_t n, int64_t k,
-                            const int64_t *group_m, const void *a, const void *b, const float *a_scale,
-                            const float *b_scale, void *out, void *stream, gg_plan **plan_out) {
-    g_last_error.clear();
-    if (plan_out == nullptr)
-        return fail(GG_ERR_INVALID, "plan_out is null");
-    *plan_out = nullptr;
+static int plan_backward(gg_plan *plan, int layout, int dtype_a, int dtype_b, int group_num, int64_t n, int64_t k,
+                         const int64_t *group_m, const void *a, const void *b, const float *a_scale,
+                         const float *b_scale, void *out) {
     if (group_num > 0 && group_m == nullptr)
         return fail(GG_ERR_INVALID, "group_m is null");
     const bool f8     = dtype_a == GG_DTYPE_FP8_E4M3 || dtype_a == GG_DTYPE_FP8_E5M2;
@@ -1331,9 +1304,6 @@ static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num,
     if (!dgrad && (rows_addr * n * es >= lim || rows_addr * k * es >= lim))
         return fail(GG_ERR_UNSUPPORTED, "one group's rows of grad_out and x must be smaller than 2 GiB");
 
-    auto *plan = new (std::nothrow) gg_plan;
-    if (plan == nullptr)
-        return fail(GG_ERR_INVALID, "out of host memory");
     plan->mode      = gg::make_mode(layout, format);
     plan->dtype     = f8 ? GG_DTYPE_BF16 : dtype_a; // output
     plan->group_num = group_num;
@@ -1345,16 +1315,13 @@ static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num,
     plan->out       = out;
 
     const int64_t n_tiles = gg::cdiv(k, gg::kTileN);
-    std::vector<gg::GroupEntry> table(static_cast<size_t>(group_num));
-    const int64_t tiles = gg::build_group_table(group_m, group_num, n_tiles, table.data(), dgrad ? 0 : n);
-    if (tiles < 0) {
-        delete plan;
+    plan->table.resize(static_cast<size_t>(group_num));
+    const int64_t tiles = gg::build_group_table(group_m, group_num, n_tiles, plan->table.data(), dgrad ? 0 : n);
+    if (tiles < 0)
         return fail(GG_ERR_UNSUPPORTED, "too many rows or tiles for 32-bit tile indices");
-    }
     // dgrad with n == 0: grad_x = 0 (gg_run zero-fills). wgrad with no rows: the tiles run and
     // store zeros (each group's K steps read nothing).
     plan->total_tiles = has_output && (!dgrad || n > 0) ? static_cast<int>(tiles) : 0;
-    const hipStream_t s = static_cast<hipStream_t>(stream);
     const std::string what = std::string(dgrad ? "dgrad" : "wgrad") +
                              (format == gg::kIn16         ? ""
                               : format == gg::kInE4M3     ? " fp8 e4m3"
@@ -1362,33 +1329,14 @@ static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num,
                                                           : " fp8 e5m2 x e4m3");
     if (plan->total_tiles > 0 && dgrad) {
         const std::string in = f8 ? "" : dtype_a == GG_DTYPE_BF16 ? " bf16" : " fp16";
-        if (use_few_rows(plan, group_m, f8 ? a_scale : nullptr, f8 ? b_scale : nullptr, what + in, s) != GG_OK) {
-            free_plan(plan);
-            return GG_ERR_HIP;
-        }
-        if (plan->few >= 0) {
-            *plan_out = plan;
-            return GG_OK;
-        }
+        if (const int st = use_few_rows(plan, group_m, f8 ? a_scale : nullptr, f8 ? b_scale : nullptr, what + in);
+            st != GG_OK || plan->few >= 0)
+            return st;
     }
     if (plan->total_tiles > 0) {
         Device dev;
-        if (current_device(&dev) != GG_OK) {
-            delete plan;
+        if (current_device(&dev) != GG_OK)
             return GG_ERR_HIP;
-        }
-        const size_t bytes = table.size() * sizeof(gg::GroupEntry);
-        hipError_t   e     = hipMalloc(&plan->d_groups, bytes);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(plan->d_groups, table.data(), bytes, hipMemcpyHostToDevice, s);
-        if (e == hipSuccess)
-            e = hipStreamSynchronize(s);
-        if (e != hipSuccess) {
-            if (plan->d_groups != nullptr)
-                (void)hipFree(plan->d_groups);
-            delete plan;
-            return hip_fail(e, "group table upload");
-        }
         plan->grid = std::min(dev.cus, plan->total_tiles);
         fill_args(plan, dev.n_xcd);
         gg::KernelArgs &ka = plan->args;
@@ -1418,25 +1366,18 @@ static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num,
             plan->total_tiles = ka.total_tiles;
             plan->detail = "mi355x " + what + " few-row 128x128 " + (f8 ? "bf16-out" : dtype_a == GG_DTYPE_BF16 ? "bf16" : "fp16") +
                            " grid=" + std::to_string(plan->grid) + " tiles=" + std::to_string(plan->total_tiles);
-            *plan_out = plan;
             return GG_OK;
         }
         // wgrad's K steps differ per group: no split
-        if (dgrad && setup_split_k(plan, dev) != GG_OK) {
-            free_plan(plan);
-            return GG_ERR_HIP;
-        }
-        if (dgrad && !f8) { // short tiles: the output rows are the groups' tokens
-            if (const int st2 = use_short_tiles(plan, group_m, s); st2 != GG_OK) {
-                free_plan(plan);
+        if (dgrad)
+            setup_split_k(plan, dev);
+        if (dgrad && !f8) // short tiles: the output rows are the groups' tokens
+            if (const int st2 = use_short_tiles(plan, group_m); st2 != GG_OK)
                 return st2;
-            }
-        }
-        if (const int st3 = setup_tile_desc(plan, group_m, s); st3 != GG_OK) {
-            free_plan(plan);
+        if (const int st3 = setup_tile_desc(plan, group_m); st3 != GG_OK)
             return st3;
-        }
-
+        if (plan->one_call)
+            return GG_OK;
         plan->detail = "mi355x " + what + " persistent " + std::to_string(ka.tile_m) + "x256x" +
                        std::to_string(f8 ? 128 : 64) + " " +
                        (f8 ? "bf16-out" : dtype_a == GG_DTYPE_BF16 ? "bf16" : "fp16") +
@@ -1447,22 +1388,17 @@ static int prepare_backward(int layout, int dtype_a, int dtype_b, int group_num,
                        (ka.splits > 1 ? " split-k=" + std::to_string(ka.splits) : "") +
                        (ka.tail_splits > 1 ? " tail-split=" + std::to_string(ka.tail_splits) : "");
     } else {
+        plan->table.clear();
         plan->detail = "mi355x " + what + ": no launch (" +
                        (has_output ? "empty contraction, zero fill" : "empty output") + ")";
         if (!has_output)
             plan->total_m = 0;
     }
-    *plan_out = plan;
     return GG_OK;
 }
 
-int gg_prepare_fp8(int dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
-                   const void *x, const void *w, const float *x_scale, const float *w_scale, void *out,
-                   void *stream, gg_plan **plan_out) {
-    g_last_error.clear();
-    if (plan_out == nullptr)
-        return fail(GG_ERR_INVALID, "plan_out is null");
-    *plan_out = nullptr;
+static int plan_fp8(gg_plan *plan, int dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
+                    const void *x, const void *w, const float *x_scale, const float *w_scale, void *out) {
     if (dtype != GG_DTYPE_FP8_E4M3 && dtype != GG_DTYPE_FP8_E5M2)
         return fail(GG_ERR_INVALID, "dtype must be GG_DTYPE_FP8_E4M3 or GG_DTYPE_FP8_E5M2");
     if (group_num > 0 && group_m == nullptr)
@@ -1488,9 +1424,6 @@ int gg_prepare_fp8(int dtype, int group_num, int64_t n, int64_t k, const int64_t
     if (k > (int64_t(1) << 21) || n > (int64_t(1) << 21))
         return fail(GG_ERR_UNSUPPORTED, "N and K must be at most 2097152");
 
-    auto *plan = new (std::nothrow) gg_plan;
-    if (plan == nullptr)
-        return fail(GG_ERR_INVALID, "out of host memory");
     plan->mode      = gg::make_mode(gg::kFwd, dtype == GG_DTYPE_FP8_E4M3 ? gg::kInE4M3 : gg::kInE5M2);
     plan->dtype     = GG_DTYPE_BF16; // output
     plan->group_num = group_num;
@@ -1501,42 +1434,18 @@ int gg_prepare_fp8(int dtype, int group_num, int64_t n, int64_t k, const int64_t
     plan->w         = w;
     plan->out       = out;
     const int64_t n_tiles = gg::cdiv(n, gg::kTileN);
-    std::vector<gg::GroupEntry> table(static_cast<size_t>(group_num));
-    const int64_t tiles = gg::build_group_table(group_m, group_num, n_tiles, table.data());
-    if (tiles < 0) {
-        delete plan;
+    plan->table.resize(static_cast<size_t>(group_num));
+    const int64_t tiles = gg::build_group_table(group_m, group_num, n_tiles, plan->table.data());
+    if (tiles < 0)
         return fail(GG_ERR_UNSUPPORTED, "too many rows or tiles for 32-bit tile indices");
-    }
     plan->total_tiles = has_output && k > 0 ? static_cast<int>(tiles) : 0;
-    const hipStream_t s = static_cast<hipStream_t>(stream);
     if (plan->total_tiles > 0) {
-        if (use_few_rows(plan, group_m, x_scale, w_scale, dtype == GG_DTYPE_FP8_E4M3 ? "fp8 e4m3" : "fp8 e5m2", s) != GG_OK) {
-            free_plan(plan);
-            return GG_ERR_HIP;
-        }
-        if (plan->few >= 0) {
-            *plan_out = plan;
-            return GG_OK;
-        }
-    }
-    if (plan->total_tiles > 0) {
+        if (const int st = use_few_rows(plan, group_m, x_scale, w_scale, dtype == GG_DTYPE_FP8_E4M3 ? "fp8 e4m3" : "fp8 e5m2");
+            st != GG_OK || plan->few >= 0)
+            return st;
         Device dev;
-        if (current_device(&dev) != GG_OK) {
-            delete plan;
+        if (current_device(&dev) != GG_OK)
             return GG_ERR_HIP;
-        }
-        const size_t bytes = table.size() * sizeof(gg::GroupEntry);
-        hipError_t   e     = hipMalloc(&plan->d_groups, bytes);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(plan->d_groups, table.data(), bytes, hipMemcpyHostToDevice, s);
-        if (e == hipSuccess)
-            e = hipStreamSynchronize(s);
-        if (e != hipSuccess) {
-            if (plan->d_groups != nullptr)
-                (void)hipFree(plan->d_groups);
-            delete plan;
-            return hip_fail(e, "group table upload");
-        }
         plan->grid = std::min(dev.cus, plan->total_tiles);
         fill_args(plan, dev.n_xcd);
         gg::KernelArgs &a = plan->args;
@@ -1546,14 +1455,11 @@ int gg_prepare_fp8(int dtype, int group_num, int64_t n, int64_t k, const int64_t
         a.tails           = k % 128 != 0;
         a.x_scale         = x_scale;
         a.w_scale         = w_scale;
-        if (setup_split_k(plan, dev) != GG_OK) {
-            free_plan(plan);
-            return GG_ERR_HIP;
-        }
-        if (const int st3 = setup_tile_desc(plan, group_m, s); st3 != GG_OK) {
-            free_plan(plan);
+        setup_split_k(plan, dev);
+        if (const int st3 = setup_tile_desc(plan, group_m); st3 != GG_OK)
             return st3;
-        }
+        if (plan->one_call)
+            return GG_OK;
         plan->detail = std::string("mi355x fp8 ") + (dtype == GG_DTYPE_FP8_E4M3 ? "e4m3" : "e5m2") +
                        " persistent 256x256x128 bf16-out grid=" + std::to_string(plan->grid) +
                        " tiles=" + std::to_string(plan->total_tiles) + " xcd=" + std::to_string(a.n_xcd) +
@@ -1562,27 +1468,37 @@ int gg_prepare_fp8(int dtype, int group_num, int64_t n, int64_t k, const int64_t
                        (a.splits > 1 ? " split-k=" + std::to_string(a.splits) : "") +
                        (a.tail_splits > 1 ? " tail-split=" + std::to_string(a.tail_splits) : "");
     } else {
+        plan->table.clear();
         plan->detail = std::string("mi355x fp8: no launch (") +
                        (has_output ? "K = 0, zero fill" : "empty output") + ")";
     }
-    *plan_out = plan;
     return GG_OK;
+}
+
+int gg_prepare_fp8(int dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
+                   const void *x, const void *w, const float *x_scale, const float *w_scale, void *out,
+                   void *stream, gg_plan **plan_out) {
+    return new_plan(plan_out, stream, [&](gg_plan *plan) {
+        return plan_fp8(plan, dtype, group_num, n, k, group_m, x, w, x_scale, w_scale, out);
+    });
 }
 
 int gg_prepare_dgrad(int dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
                      const void *grad_out, const void *w, void *grad_x, void *stream, gg_plan **plan_out) {
     if (dtype != GG_DTYPE_BF16 && dtype != GG_DTYPE_FP16)
         return fail(GG_ERR_INVALID, "dtype must be GG_DTYPE_BF16 or GG_DTYPE_FP16");
-    return prepare_backward(gg::kDgrad, dtype, dtype, group_num, n, k, group_m, grad_out, w, nullptr, nullptr,
-                            grad_x, stream, plan_out);
+    return new_plan(plan_out, stream, [&](gg_plan *plan) {
+        return plan_backward(plan, gg::kDgrad, dtype, dtype, group_num, n, k, group_m, grad_out, w, nullptr, nullptr, grad_x);
+    });
 }
 
 int gg_prepare_wgrad(int dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
                      const void *grad_out, const void *x, void *grad_w, void *stream, gg_plan **plan_out) {
     if (dtype != GG_DTYPE_BF16 && dtype != GG_DTYPE_FP16)
         return fail(GG_ERR_INVALID, "dtype must be GG_DTYPE_BF16 or GG_DTYPE_FP16");
-    return prepare_backward(gg::kWgrad, dtype, dtype, group_num, n, k, group_m, grad_out, x, nullptr, nullptr,
-                            grad_w, stream, plan_out);
+    return new_plan(plan_out, stream, [&](gg_plan *plan) {
+        return plan_backward(plan, gg::kWgrad, dtype, dtype, group_num, n, k, group_m, grad_out, x, nullptr, nullptr, grad_w);
+    });
 }
 
 int gg_prepare_dgrad_fp8(int grad_dtype, int w_dtype, int group_num, int64_t n, int64_t k,
@@ -1590,8 +1506,9 @@ int gg_prepare_dgrad_fp8(int grad_dtype, int w_dtype, int group_num, int64_t n, 
                          const float *w_scale, void *grad_x, void *stream, gg_plan **plan_out) {
     if (grad_dtype != GG_DTYPE_FP8_E4M3 && grad_dtype != GG_DTYPE_FP8_E5M2)
         return fail(GG_ERR_INVALID, "grad_dtype must be GG_DTYPE_FP8_E4M3 or GG_DTYPE_FP8_E5M2");
-    return prepare_backward(gg::kDgrad, grad_dtype, w_dtype, group_num, n, k, group_m, grad_out, w, grad_scale,
-                            w_scale, grad_x, stream, plan_out);
+    return new_plan(plan_out, stream, [&](gg_plan *plan) {
+        return plan_backward(plan, gg::kDgrad, grad_dtype, w_dtype, group_num, n, k, group_m, grad_out, w, grad_scale, w_scale, grad_x);
+    });
 }
 
 int gg_prepare_wgrad_fp8(int grad_dtype, int x_dtype, int group_num, int64_t n, int64_t k,
@@ -1599,8 +1516,9 @@ int gg_prepare_wgrad_fp8(int grad_dtype, int x_dtype, int group_num, int64_t n, 
                          const float *x_scale, void *grad_w, void *stream, gg_plan **plan_out) {
     if (grad_dtype != GG_DTYPE_FP8_E4M3 && grad_dtype != GG_DTYPE_FP8_E5M2)
         return fail(GG_ERR_INVALID, "grad_dtype must be GG_DTYPE_FP8_E4M3 or GG_DTYPE_FP8_E5M2");
-    return prepare_backward(gg::kWgrad, grad_dtype, x_dtype, group_num, n, k, group_m, grad_out, x, grad_scale,
-                            x_scale, grad_w, stream, plan_out);
+    return new_plan(plan_out, stream, [&](gg_plan *plan) {
+        return plan_backward(plan, gg::kWgrad, grad_dtype, x_dtype, group_num, n, k, group_m, grad_out, x, grad_scale, x_scale, grad_w);
+    });
 }
 
 int gg_prepare_device_lens(int dtype, int group_num, int64_t total_m, int64_t n, int64_t k,
@@ -1628,7 +1546,7 @@ int gg_prepare_device_lens_op(int op, int a_dtype, int b_dtype, int group_num, i
     auto *plan = new (std::nothrow) gg_plan;
     if (plan == nullptr)
         return fail(GG_ERR_INVALID, "out of host memory");
-    const int st = plan_device_lens(plan, false, op, a_dtype, b_dtype, group_num, total_m, n, k, group_lens,
+    const int st = plan_device_lens(plan, kOwned, nullptr, op, a_dtype, b_dtype, group_num, total_m, n, k, group_lens,
                                     group_offs, a, b, a_scale, b_scale, out);
     if (st != GG_OK) {
         free_plan(plan);
@@ -1648,11 +1566,94 @@ int gg_run_device_lens_noalloc(int op, int a_dtype, int b_dtype, int group_num, 
                                             std::to_string(kNoAllocMaxGroups) + " groups (got " +
                                             std::to_string(group_num) + ")");
     gg_plan plan; // on the stack: its table is the device's scratch array
-    const int st = plan_device_lens(&plan, true, op, a_dtype, b_dtype, group_num, total_m, n, k, group_lens,
+    const int st = plan_device_lens(&plan, kScratch, nullptr, op, a_dtype, b_dtype, group_num, total_m, n, k, group_lens,
                                     group_offs, a, b, a_scale, b_scale, out);
     if (st != GG_OK)
         return st;
     return run_plan(&plan, stream, true);
+}
+
+// What a run's table header says about its device sizes.
+static int check_header(const gg::TableHeader &h) {
+    if (h.overflow != 0)
+        return fail(GG_ERR_INVALID, "device group sizes: more than 2^31 tiles, nothing computed");
+    if (h.first_bad >= 0)
+        return fail(GG_ERR_INVALID, "device group sizes: group " + std::to_string(h.first_bad) +
+                                        " has a negative length or rows outside [0, total_m); "
+                                        "its rows were not written");
+    return GG_OK;
+}
+
+int gg_call(int op, int a_dtype, int b_dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
+            const void *a, const void *b, const float *a_scale, const float *b_scale, void *out,
+            void *workspace, size_t workspace_bytes, size_t *needed, void *stream) {
+    g_last_error.clear();
+    if (needed == nullptr)
+        return fail(GG_ERR_INVALID, "needed is null");
+    *needed = 0;
+    if (op != GG_OP_FORWARD && op != GG_OP_DGRAD && op != GG_OP_WGRAD)
+        return fail(GG_ERR_INVALID, "op must be GG_OP_FORWARD, GG_OP_DGRAD or GG_OP_WGRAD");
+    const bool f8 = a_dtype == GG_DTYPE_FP8_E4M3 || a_dtype == GG_DTYPE_FP8_E5M2;
+    if (op == GG_OP_FORWARD && a_dtype != b_dtype)
+        return fail(GG_ERR_INVALID, "x and w must have one dtype");
+    gg_plan plan; // on the stack: its device memory is the caller's workspace
+    plan.one_call = true;
+    const int st  = op != GG_OP_FORWARD ? plan_backward(&plan, op == GG_OP_DGRAD ? gg::kDgrad : gg::kWgrad, a_dtype, b_dtype,
+                                                        group_num, n, k, group_m, a, b, a_scale, b_scale, out)
+                    : f8 ? plan_fp8(&plan, a_dtype, group_num, n, k, group_m, a, b, a_scale, b_scale, out)
+                         : plan_forward(&plan, a_dtype, group_num, n, k, group_m, a, b, out);
+    if (st != GG_OK)
+        return st;
+    *needed = plan_bytes(&plan);
+    if (*needed > workspace_bytes)
+        return fail(GG_ERR_WORKSPACE, "workspace of " + std::to_string(workspace_bytes) + " bytes, " +
+                                          std::to_string(*needed) + " needed");
+    if (*needed > 0 && (workspace == nullptr || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0))
+        return fail(GG_ERR_INVALID, "workspace must be 256-byte aligned device memory");
+    if (*needed > 0) {
+        std::vector<char> image;
+        bind_plan(&plan, workspace, &image);
+        const hipError_t e = gg::launch_upload(workspace, image.data(), image.size(), static_cast<hipStream_t>(stream));
+        if (e != hipSuccess)
+            return hip_fail(e, "plan table upload");
+    }
+    return run_plan(&plan, stream, true);
+}
+
+int gg_call_device_lens(int op, int a_dtype, int b_dtype, int group_num, int64_t total_m, int64_t n, int64_t k,
+                        const int64_t *group_lens, const int64_t *group_offs, const void *a, const void *b,
+                        const float *a_scale, const float *b_scale, void *out, void *workspace,
+                        size_t workspace_bytes, void *status, void *stream) {
+    g_last_error.clear();
+    if (status == nullptr)
+        return fail(GG_ERR_INVALID, "status is null");
+    auto *header = static_cast<gg::TableHeader *>(status);
+    *header      = gg::TableHeader{0, -1, 0, 0};
+    if (group_num > 0 && (workspace == nullptr || workspace_bytes < device_table_bytes(group_num) ||
+                          (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0))
+        return fail(GG_ERR_INVALID, "workspace must be 16 * (group_num + 1) bytes of 256-byte aligned device memory");
+    gg_plan plan;
+    int     st = plan_device_lens(&plan, kGiven, workspace, op, a_dtype, b_dtype, group_num, total_m, n, k, group_lens,
+                                  group_offs, a, b, a_scale, b_scale, out);
+    if (st != GG_OK)
+        return st;
+    if (plan.in_kernel_table) // the GEMM writes the header once, straight to the host
+        plan.args.d_header = header;
+    st = run_plan(&plan, stream, true);
+    if (st == GG_OK && plan.d_header != nullptr && !plan.in_kernel_table) {
+        const hipError_t e = hipMemcpyAsync(status, plan.d_header, sizeof(gg::TableHeader), hipMemcpyDeviceToHost,
+                                            static_cast<hipStream_t>(stream));
+        if (e != hipSuccess)
+            return hip_fail(e, "device status read");
+    }
+    return st;
+}
+
+int gg_check_status(const void *status) {
+    g_last_error.clear();
+    if (status == nullptr)
+        return fail(GG_ERR_INVALID, "status is null");
+    return check_header(*static_cast<const gg::TableHeader *>(status));
 }
 
 int gg_run(const gg_plan *plan, void *stream) {
@@ -1691,13 +1692,7 @@ int gg_plan_device_status(const gg_plan *plan, void *stream, int *total_tiles) {
         return hip_fail(e, "device status read");
     if (total_tiles != nullptr)
         *total_tiles = h.total_tiles;
-    if (h.overflow != 0)
-        return fail(GG_ERR_INVALID, "device group sizes: more than 2^31 tiles, nothing computed");
-    if (h.first_bad >= 0)
-        return fail(GG_ERR_INVALID, "device group sizes: group " + std::to_string(h.first_bad) +
-                                        " has a negative length or rows outside [0, total_m); "
-                                        "its rows were not written");
-    return GG_OK;
+    return check_header(h);
 }
 
 int gg_compute_group_offs(const int64_t *group_lens, int64_t *group_offs, int group_num,

@@ -192,6 +192,12 @@ struct SmallArgs {
 // reduction of the partial sums, one workgroup of 256 threads per tile, on the same stream.
 hipError_t launch_small_gemm(const SmallArgs &args, bool fp16, hipStream_t stream);
 
+// Copies `bytes` (a multiple of 16) of host memory to 16-byte aligned device memory on `stream`: the
+// bytes travel in kernel arguments, so `src` may be freed at once and nothing is waited for (more
+// than kUploadMaxBytes: a copy that is waited for).
+constexpr size_t kUploadMaxBytes = 32768;
+hipError_t launch_upload(void *dst, const void *src, size_t bytes, hipStream_t stream);
+
 // Seeded N(0,1) fill (benchmark input generator).
 hipError_t launch_fill_randn(void *p, size_t count, uint64_t seed, bool fp16, hipStream_t stream);
 hipError_t launch_clock_probe(unsigned long long *out, unsigned long long ticks, unsigned long long wall_hz,

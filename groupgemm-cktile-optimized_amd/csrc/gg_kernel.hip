@@ -4,6 +4,9 @@
 // build runs in parallel.
 #include "gg_kernel_impl.h"
 
+#include <algorithm>
+#include <cstring>
+
 namespace gg {
 namespace {
 
@@ -153,6 +156,16 @@ __global__ void __launch_bounds__(256) zero_fill_kernel(u32x4 *out, size_t n16) 
     const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
     for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < n16; i += stride)
         out[i] = u32x4{0u, 0u, 0u, 0u};
+}
+
+// Bytes that travel as kernel arguments (launch_upload).
+template <int N> struct Payload {
+    u32x4 v[N];
+};
+template <int N> __global__ void __launch_bounds__(N) upload_kernel(u32x4 *dst, const Payload<N> p, int n16) {
+    const int i = static_cast<int>(threadIdx.x);
+    if (i < n16)
+        dst[i] = p.v[i];
 }
 
 // ---------------------------------------------------------------------------------------
@@ -335,6 +348,36 @@ hipError_t launch_zero_fill(void *out, size_t bytes, hipStream_t stream) {
     const size_t blocks = std::min<size_t>((n16 + 255) / 256, 4096);
     hipLaunchKernelGGL(zero_fill_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
                        static_cast<u32x4 *>(out), n16);
+    return hipGetLastError();
+}
+
+template <int N> void upload_part(char *dst, const char *src, size_t bytes, hipStream_t stream) {
+    Payload<N> p{};
+    std::memcpy(&p, src, bytes);
+    hipLaunchKernelGGL(upload_kernel<N>, dim3(1), dim3(N), 0, stream, reinterpret_cast<u32x4 *>(dst), p,
+                       static_cast<int>(bytes / 16));
+}
+
+hipError_t launch_upload(void *dst, const void *src, size_t bytes, hipStream_t stream) {
+    if (bytes % 16 != 0 || (reinterpret_cast<uintptr_t>(dst) & 15u) != 0)
+        return hipErrorInvalidValue;
+    if (bytes > kUploadMaxBytes) {
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
+        return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+    }
+    // 3.5 KB of arguments at most per launch (64 groups' table is 1 KB)
+    for (size_t at = 0; at < bytes;) {
+        const size_t left = bytes - at, part = left < 3584 ? left : 3584;
+        char        *d    = static_cast<char *>(dst) + at;
+        const char  *f    = static_cast<const char *>(src) + at;
+        if (part <= 256)
+            upload_part<16>(d, f, part, stream);
+        else if (part <= 1024)
+            upload_part<64>(d, f, part, stream);
+        else
+            upload_part<224>(d, f, part, stream);
+        at += part;
+    }
     return hipGetLastError();
 }
 

@@ -46,7 +46,9 @@ typedef enum gg_status {
     GG_ERR_INVALID = 2,
     /* A HIP runtime call failed (the reference's TUNEMAX_HIP_CHECK, common/backend.hpp:15-23,
      * prints and exits; this library returns the code and keeps the message). */
-    GG_ERR_HIP = 3
+    GG_ERR_HIP = 3,
+    /* gg_call: the workspace is too small; nothing was enqueued and *needed says how much it takes. */
+    GG_ERR_WORKSPACE = 4
 } gg_status;
 
 /* Opaque per-problem plan: device group table, launch shape, pointers. */
@@ -226,6 +228,31 @@ int gg_run_device_lens_noalloc(int op, int a_dtype, int b_dtype, int group_num, 
                                int64_t k, const int64_t *group_lens, const int64_t *group_offs, const void *a,
                                const void *b, const float *a_scale, const float *b_scale, void *out,
                                void *stream);
+
+/*
+ * A prepare, run and release of host-size groups in one call on `stream`, in the caller's device
+ * memory: nothing is allocated, freed or waited for. op, a, b, out and the scales as in
+ * gg_prepare_device_lens_op, group_m and the requirements as in the matching host-size prepare
+ * (gg_prepare, gg_prepare_fp8, gg_prepare_dgrad, ...). workspace: workspace_bytes of 256-byte
+ * aligned device memory that must stay valid until the work on `stream` is done; if that is too
+ * little, GG_ERR_WORKSPACE comes back with the size in *needed and nothing is enqueued. (Group tables
+ * take 16 bytes per group; split-K partial sums up to 64 MB.) No counterpart in the reference.
+ */
+int gg_call(int op, int a_dtype, int b_dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
+            const void *a, const void *b, const float *a_scale, const float *b_scale, void *out,
+            void *workspace, size_t workspace_bytes, size_t *needed, void *stream);
+
+/*
+ * The same over device-resident sizes (gg_prepare_device_lens_op): workspace of at least
+ * 16 * (group_num + 1) bytes of 256-byte aligned device memory. status: 16 bytes of pinned host
+ * memory that the run fills; once the work on `stream` is done, gg_check_status(status) reports
+ * sizes that did not fit, as gg_plan_device_status does for a plan.
+ */
+int gg_call_device_lens(int op, int a_dtype, int b_dtype, int group_num, int64_t total_m, int64_t n, int64_t k,
+                        const int64_t *group_lens, const int64_t *group_offs, const void *a, const void *b,
+                        const float *a_scale, const float *b_scale, void *out, void *workspace,
+                        size_t workspace_bytes, void *status, void *stream);
+int gg_check_status(const void *status);
 
 /* Message of the last failed call on the calling thread ("" if none). */
 const char *gg_last_error(void);
