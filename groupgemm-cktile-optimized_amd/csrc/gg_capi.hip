@@ -14,6 +14,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -796,6 +797,15 @@ int setup_tile_desc(gg_plan *plan, const int64_t *group_m) {
     const int64_t tiles = gg::build_group_table(group_m, plan->group_num, a.n_tiles, table.data(), out_rows, a.tile_m);
     if (tiles != plan->total_tiles)
         return fail(GG_ERR_INVALID, "tile descriptors: the group table's tile count differs from the plan's");
+    // wgrad groups are walked by descending K steps, every other round backwards (snake_slot), so
+    // that ragged groups load the workgroups evenly; equal groups keep their own order
+    std::vector<int> order(static_cast<size_t>(plan->group_num));
+    std::iota(order.begin(), order.end(), 0);
+    if (wgrad) {
+        const int rows_per = plan->mode / 4 == gg::kIn16 ? gg::kTileK : 128;
+        const auto steps   = [&](int g) { return std::max<int64_t>(gg::kCrossMinStepsHost, gg::cdiv(group_m[g], rows_per)); };
+        std::stable_sort(order.begin(), order.end(), [&](int l, int r) { return steps(l) > steps(r); });
+    }
     std::vector<gg::TileDesc> desc(static_cast<size_t>(plan->grid) * per_wg, gg::TileDesc{0, 0, 0, 0});
     for (int wg = 0; wg < plan->grid; ++wg) {
         int g = 0; // locate_tile's hint: a workgroup's logical tiles only grow
@@ -803,13 +813,15 @@ int setup_tile_desc(gg_plan *plan, const int64_t *group_m) {
             const int t = wg + i * plan->grid;
             if (t >= plan->total_tiles)
                 break;
-            const int L = gg::xcd_remap(t, plan->total_tiles, plan->grid, a.n_xcd);
+            const int slot = wgrad ? gg::snake_slot(t, plan->total_tiles, plan->grid) : t;
+            const int L    = gg::xcd_remap(slot, plan->total_tiles, plan->grid, a.n_xcd);
             int       tm, tn;
             gg::locate_tile(L, table.data(), plan->group_num, a.n_tiles, a.band, &g, &tm, &tn,
                             static_cast<int>(out_rows), a.tile_m);
             if (wgrad) { // the group's first token, (N-tile << 16) | M-tile, the group's tokens
+                const int og = order[static_cast<size_t>(g)];
                 desc[static_cast<size_t>(wg) * per_wg + i] =
-                    gg::TileDesc{static_cast<int32_t>(table[g].row0), g, (tn << 16) | tm, table[g].m};
+                    gg::TileDesc{static_cast<int32_t>(table[og].row0), og, (tn << 16) | tm, table[og].m};
                 continue;
             }
             const int64_t r0 = table[g].row0 + static_cast<int64_t>(tm) * a.tile_m;

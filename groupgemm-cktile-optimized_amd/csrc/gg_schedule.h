@@ -58,6 +58,15 @@ GG_HD int xcd_remap(int t, int total, int grid, int n_xcd) {
     return base + before + local;
 }
 
+// Slot t of a wgrad launch whose groups are walked by descending K steps: whole odd rounds run
+// backwards, so a workgroup that drew one of a round's longest tiles draws one of the next round's
+// shortest (boustrophedon); the last, partial round keeps its slots. A bijection of each round's
+// slots, so a workgroup's logical tiles still grow from round to round.
+GG_HD int snake_slot(int t, int total, int grid) {
+    const int round = t / grid, base = round * grid;
+    return (round & 1) != 0 && total - base >= grid ? base + grid - 1 - (t - base) : t;
+}
+
 // (M-tile, N-tile) of the tile at position `local` inside a group with m_tiles x n_tiles
 // tiles, in the banded order described above.
 GG_HD void band_coords(int local, int m_tiles, int n_tiles, int band, int *tm, int *tn) {

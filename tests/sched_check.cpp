@@ -205,8 +205,24 @@ static void check_desc_rows() {
     CHECK(gg::desc_rows_fit(nullptr, 0, 0), "an empty plan fits");
 }
 
+// snake_slot permutes each whole round's slots, leaves even and partial rounds alone, and undoes itself.
+static void check_snake(int total, int grid) {
+    std::set<int> seen;
+    for (int t = 0; t < total; ++t) {
+        const int s = gg::snake_slot(t, total, grid), round = t / grid;
+        CHECK(s / grid == round && s < total && seen.insert(s).second, "slot %d -> %d of %d, grid %d", t, s, total, grid);
+        CHECK(gg::snake_slot(s, total, grid) == t, "slot %d not undone", t);
+        if (round % 2 == 0 || (round + 1) * grid > total)
+            CHECK(s == t, "slot %d moved to %d", t, s);
+    }
+}
+
 int main() {
     check_desc_rows();
+    for (int grid : {1, 3, 8, 256})
+        for (int total = 1; total <= 1300; total += (total < 20 ? 1 : 61))
+            check_snake(total, grid);
+    check_snake(1024, 256);
     check_short(std::vector<int64_t>(32, 520), 2880, 176); // config 5a: 3 x 176 instead of 256 + 256 + 8
     check_short({300, 0, 260, 130}, 1000, 160);
     check_short({100, 7, 1}, 264, 112);
