@@ -105,6 +105,13 @@ int check_problem(int dtype, int group_num, int64_t n, int64_t k, bool has_outpu
     return GG_OK;
 }
 
+// Whether a problem runs on the instances of its own formats. An fp8 one that reads nothing may come
+// without scales (wgrad of groups without rows: every tile runs and stores zeros), and the fp8 instances
+// load the scales whatever the rows: those zeros come from the 16-bit instance, which loads none.
+bool own_format(bool f8, bool reads, const float *a_scale, const float *b_scale) {
+    return !f8 || reads || (a_scale != nullptr && b_scale != nullptr);
+}
+
 // Launch facts of the current device, queried from the runtime on the device's first use.
 struct Device {
     int cus   = 0;
@@ -949,7 +956,7 @@ int plan_device_lens(gg_plan *plan, TableMemory memory, void *given, int op, int
     if (wgrad_tiles > INT32_MAX)
         return fail(GG_ERR_UNSUPPORTED, "too many tiles for 32-bit tile indices");
 
-    plan->mode        = gg::make_mode(layout, format);
+    plan->mode        = gg::make_mode(layout, own_format(f8, reads, a_scale, b_scale) ? format : gg::kIn16);
     plan->dtype       = f8 ? GG_DTYPE_BF16 : a_dtype; // output
     plan->group_num   = group_num;
     plan->n           = n_out;
@@ -1316,7 +1323,7 @@ static int plan_backward(gg_plan *plan, int layout, int dtype_a, int dtype_b, in
     if (!dgrad && (rows_addr * n * es >= lim || rows_addr * k * es >= lim))
         return fail(GG_ERR_UNSUPPORTED, "one group's rows of grad_out and x must be smaller than 2 GiB");
 
-    plan->mode      = gg::make_mode(layout, format);
+    plan->mode      = gg::make_mode(layout, own_format(f8, reads, a_scale, b_scale) ? format : gg::kIn16);
     plan->dtype     = f8 ? GG_DTYPE_BF16 : dtype_a; // output
     plan->group_num = group_num;
     plan->n         = k;                      // output columns
