@@ -637,10 +637,11 @@ int choose_few_rows(const gg_plan *plan, const int64_t *group_m, int64_t rows, i
     double       least = kFewGain * other;
     for (int i = 0; i < gg::kFewInstanceCount; ++i) {
         const gg::FewInstance &f = gg::kFewInstances[i];
-        // (device sizes may put every row in each group: the count must fit 32 bits even then)
-        const int64_t nt = gg::cdiv(plan->n, f.tile_n);
-        if (forced >= 0 ? i != forced
-                        : double(plan->group_num) * double(gg::cdiv(rows, f.tile_m)) * double(nt) > double(INT32_MAX))
+        // the kernel's tile index must not pass 2^31 (device sizes may put every row in each group)
+        const int64_t nt   = gg::cdiv(plan->n, f.tile_n);
+        const double  most = group_m != nullptr ? row_tiles(group_m, plan->group_num, rows, f.tile_m)
+                                                : double(plan->group_num) * double(gg::cdiv(rows, f.tile_m));
+        if ((forced >= 0 && i != forced) || most * double(nt) > double(gg::kMaxLoopTiles))
             continue;
         const double wgs    = row_tiles(group_m, plan->group_num, rows, f.tile_m) * nt;
         const double staged = wgs * (f.tile_m + f.tile_n) * 128.0 * chunks;
@@ -676,7 +677,7 @@ void few_args(gg_plan *plan, int64_t tiles) {
         a.lda = static_cast<int>(plan->k);
         a.ldb = static_cast<int>(plan->n);
     }
-    plan->grid = static_cast<int>(gg::cdiv(std::min<int64_t>(tiles, 1 << 20), 8) * 8);
+    plan->grid = static_cast<int>(gg::cdiv(std::min<int64_t>(tiles, gg::kMaxLoopGrid), 8) * 8);
 }
 
 std::string few_detail(const gg_plan *plan, const std::string &what) {
@@ -704,11 +705,15 @@ std::string few_detail(const gg_plan *plan, const std::string &what) {
 constexpr double kWgradFewGain = 0.9, kWgradFewFixedUs = 3.7, kWgradFixedUs = 7.8; // us
 constexpr double kWgradFewHbm = 6.1e6, kWgradHbm = 5.1e6;                          // bytes per us
 
+int64_t wgrad_few_tiles(const gg_plan *plan, int64_t m_out) {
+    return int64_t(plan->group_num) * gg::cdiv(m_out, gg::kWgradFewTile) * gg::cdiv(plan->n, gg::kWgradFewTile);
+}
+
 bool choose_wgrad_few(const gg_plan *plan, const int64_t *group_m, int64_t m_out, int64_t rows, int cus) {
     if (const char *env = std::getenv("GG_SMALL"); env != nullptr && *env != '\0')
         return false;
-    const double tiles = double(plan->group_num) * gg::cdiv(m_out, gg::kWgradFewTile) * gg::cdiv(plan->n, gg::kWgradFewTile);
-    if (tiles > INT32_MAX - 64)
+    const double tiles = static_cast<double>(wgrad_few_tiles(plan, m_out));
+    if (gg::one_tile_grid(wgrad_few_tiles(plan, m_out), gg::kWgradFewThreads) == 0)
         return false;
     if (const char *env = std::getenv("GG_WFEW"); env != nullptr && *env != '\0')
         return std::atoi(env) != 0;
@@ -739,12 +744,11 @@ bool choose_wgrad_few(const gg_plan *plan, const int64_t *group_m, int64_t m_out
 // rows of a group's gradient).
 void wgrad_few_args(gg_plan *plan, int64_t m_out, int n_xcd) {
     gg::KernelArgs &a = plan->args;
-    a.total_tiles     = static_cast<int>(int64_t(plan->group_num) * gg::cdiv(m_out, gg::kWgradFewTile) *
-                                         gg::cdiv(plan->n, gg::kWgradFewTile));
+    a.total_tiles     = static_cast<int>(wgrad_few_tiles(plan, m_out));
     a.m_out           = static_cast<int>(m_out);
     a.d_total         = nullptr;
     plan->wgrad_few   = true;
-    plan->grid        = static_cast<int>(gg::cdiv(a.total_tiles, 8) * 8);
+    plan->grid        = static_cast<int>(gg::one_tile_grid(a.total_tiles, gg::kWgradFewThreads));
     a.n_xcd           = plan->grid % n_xcd == 0 ? n_xcd : 1;
 }
 

@@ -32,7 +32,7 @@ hipError_t launch_few_gemm(const KernelArgs &args, int format, bool mn, int inst
 
 // The 128 x 128 wgrad kernel (gg_wfew.hip): one workgroup per tile, `grid` of at least
 // args.total_tiles of them (group by group: ceil(m_out / 128) x ceil(n / 128) each).
-constexpr int kWgradFewTile = 128;
+constexpr int kWgradFewTile = 128, kWgradFewThreads = 256;
 hipError_t launch_wgrad_few(const KernelArgs &args, int format, int grid, hipStream_t stream);
 
 } // namespace gg

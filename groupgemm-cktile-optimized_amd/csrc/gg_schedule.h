@@ -58,6 +58,17 @@ GG_HD int xcd_remap(int t, int total, int grid, int n_xcd) {
     return base + before + local;
 }
 
+// Workgroups of a launch of one workgroup of `threads` threads per tile, in whole rows of 8 XCDs; 0 if the
+// launch takes none: HIP refuses grids of 2^32 threads and more.
+GG_HD int64_t one_tile_grid(int64_t tiles, int threads) {
+    const int64_t grid = (tiles + 7) / 8 * 8;
+    return grid > UINT32_MAX / threads ? 0 : grid;
+}
+
+// Tiles that a launch of at most kMaxLoopGrid workgroups walks by t += grid without passing 2^31.
+constexpr int64_t kMaxLoopGrid  = int64_t(1) << 20;
+constexpr int64_t kMaxLoopTiles = INT32_MAX - kMaxLoopGrid;
+
 // Slot t of a wgrad launch whose groups are walked by descending K steps: whole odd rounds run
 // backwards, so a workgroup that drew one of a round's longest tiles draws one of the next round's
 // shortest (boustrophedon); the last, partial round keeps its slots. A bijection of each round's

@@ -35,7 +35,7 @@ constexpr int kWT = kWgradFewTile; // 128 x 128 outputs per workgroup
 constexpr int kWRow = 272;         // staged output row stride (256 bytes + 16)
 
 template <int FMT, int R, int S, int OCC>
-__global__ void __launch_bounds__(256, OCC) wgrad_few_kernel(const KernelArgs args) {
+__global__ void __launch_bounds__(kWgradFewThreads, OCC) wgrad_few_kernel(const KernelArgs args) {
     constexpr bool kF8   = FMT >= kFewE4M3;
     constexpr bool kF16  = FMT == kFewF16;
     constexpr int  es    = kF8 ? 1 : 2;
@@ -217,7 +217,8 @@ __global__ void __launch_bounds__(256, OCC) wgrad_few_kernel(const KernelArgs ar
 
 template <int FMT> void launch_format(const KernelArgs &a, int grid, hipStream_t s) {
     constexpr bool f8 = FMT >= kFewE4M3;
-    hipLaunchKernelGGL((wgrad_few_kernel<FMT, f8 ? 128 : 32, f8 ? 1 : 2, 4>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((wgrad_few_kernel<FMT, f8 ? 128 : 32, f8 ? 1 : 2, 4>), dim3(static_cast<unsigned>(grid)),
+                       dim3(kWgradFewThreads), 0, s, a);
 }
 
 hipError_t launch_wgrad_few(const KernelArgs &a, int format, int grid, hipStream_t s) {

@@ -13,7 +13,8 @@
 //   * band_for: 8-tile bands exactly where one group's B operand passes the Infinity Cache;
 //   * desc_rows_fit: tile descriptors (32-bit first rows) are refused when a wgrad plan's input
 //     tokens pass 2^31 although its output rows (group_num * N) are few, and accepted when every
-//     group's first token from build_group_table fits.
+//     group's first token from build_group_table fits;
+//   * one_tile_grid and kMaxLoopTiles: launches and tile indices stay inside 32 bits.
 #include <cstdio>
 #include <cstdlib>
 #include <set>
@@ -277,6 +278,13 @@ int main() {
     check_walk({16384}, 32768, 256, 8, 0, gg::kTileM, gg::kBandWide);
     check_walk({0, 300, 0, 0, 1, 2000, 0}, 1000, 24, 8, 0, gg::kTileM, gg::kBandWide);
     check_walk({257, 0, 255, 4096, 3}, 264, 256, 8, 0, gg::kTileM, gg::kBandWide);
+    // launches of one workgroup per tile: whole rows of 8, refused from 2^32 threads on (2^24 tiles of 256)
+    CHECK(gg::one_tile_grid(1, 256) == 8 && gg::one_tile_grid(16, 256) == 16, "grids of whole XCD rows");
+    CHECK(gg::one_tile_grid((1 << 24) - 8, 256) == (1 << 24) - 8, "the largest grid is refused");
+    CHECK(gg::one_tile_grid((1 << 24) - 7, 256) == 0, "2^32 threads are not refused");
+    CHECK(gg::one_tile_grid(int64_t(1) << 59, 256) == 0, "2^59 tiles are not refused");
+    // walks by t += grid: the last index looked at is below 2^31
+    CHECK(gg::kMaxLoopTiles - 1 + gg::kMaxLoopGrid < INT32_MAX, "tile index past 2^31");
     if (failures) {
         std::printf("%d failures\n", failures);
         return 1;

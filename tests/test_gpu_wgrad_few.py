@@ -170,3 +170,20 @@ def test_fp8_gradients_of_no_rows_need_no_scales(pkg, monkeypatch, few, device):
     assert ("few-row" in plan.detail()) == few, plan.detail()
     zeros(lambda: plan.run(_stream()))
     plan.release()
+
+
+def test_more_tiles_than_one_launch_takes(pkg, monkeypatch):
+    """2^24 groups of one tile each: a launch of one workgroup per tile would pass HIP's 2^32 threads, so the
+    persistent kernel runs, also where the 128 x 128 one is asked for."""
+    monkeypatch.delenv("GG_SMALL", raising=False)
+    monkeypatch.setenv("GG_WFEW", "1")
+    lib, b, plan = pkg.load_library(), 1 << 24, ctypes.c_void_p()
+    out = torch.ones((b, 8, 8), dtype=torch.bfloat16, device=DEV)
+    st = lib.gg_prepare_wgrad(int(pkg.DType.BF16), b, 8, 8, (ctypes.c_int64 * b)(), 0, 0, out.data_ptr(), _stream(),
+                              ctypes.byref(plan))
+    assert st == pkg.GG_OK, pkg.last_error()
+    assert "persistent" in lib.gg_plan_detail(plan).decode()
+    assert lib.gg_run(plan, _stream()) == pkg.GG_OK, pkg.last_error()
+    torch.cuda.synchronize(DEV)
+    lib.gg_release(plan)
+    assert torch.count_nonzero(out) == 0
