@@ -409,11 +409,15 @@ def _call_device(op: int, a_dtype: DType, b_dtype: DType, n: int, k: int, group_
     ws = torch.empty(16 * (count + 1), dtype=torch.uint8, device=a.device)
     status = torch.empty(4, dtype=torch.int32, pin_memory=True)
     sa, sb = (0, 0) if a_scale is None else (a_scale.data_ptr(), b_scale.data_ptr())
-    _check(lib.gg_call_device_lens(op, int(a_dtype), int(b_dtype), count, rows, n, k, group_lens.data_ptr(),
-                                   0 if group_offs is None else group_offs.data_ptr(), a.data_ptr(), b.data_ptr(),
-                                   sa, sb, out.data_ptr(), ws.data_ptr(), ws.numel(), status.data_ptr(),
-                                   stream.cuda_stream))
-    stream.synchronize()
+    try:
+        _check(lib.gg_call_device_lens(op, int(a_dtype), int(b_dtype), count, rows, n, k, group_lens.data_ptr(),
+                                       0 if group_offs is None else group_offs.data_ptr(), a.data_ptr(), b.data_ptr(),
+                                       sa, sb, out.data_ptr(), ws.data_ptr(), ws.numel(), status.data_ptr(),
+                                       stream.cuda_stream))
+    finally:
+        # also where the call failed or was interrupted: what it enqueued writes status, whose memory
+        # torch gives to the next caller without waiting for this stream
+        stream.synchronize()
     _check(lib.gg_check_status(status.data_ptr()))
 
 
