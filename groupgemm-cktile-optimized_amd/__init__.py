@@ -407,7 +407,7 @@ def _call_device(op: int, a_dtype: DType, b_dtype: DType, n: int, k: int, group_
     lib, count = load_library(), group_lens.numel()
     stream = torch.cuda.current_stream(a.device)
     ws = torch.empty(16 * (count + 1), dtype=torch.uint8, device=a.device)
-    status = torch.empty(4, dtype=torch.int32, pin_memory=True)
+    status = torch.empty(4, dtype=torch.int32, device="cpu", pin_memory=True)  # (whatever the default device)
     sa, sb = (0, 0) if a_scale is None else (a_scale.data_ptr(), b_scale.data_ptr())
     try:
         _check(lib.gg_call_device_lens(op, int(a_dtype), int(b_dtype), count, rows, n, k, group_lens.data_ptr(),

@@ -18,10 +18,13 @@ class _Stream:
 
 def _run(pkg, monkeypatch, call):
     """_call_device over CPU tensors with `call` as gg_call_device_lens; returns the stream."""
-    stream, empty = _Stream(), torch.empty
+    stream, pinned, empty = _Stream(), [], torch.empty
 
     def empty_without_pinning(*shape, pin_memory=False, **kw):
-        return empty(*shape, **kw)
+        t = empty(*shape, **kw)
+        if pin_memory:
+            pinned.append(t)
+        return t
 
     lib = types.SimpleNamespace(gg_call_device_lens=call, gg_check_status=lambda p: pkg.GG_OK)
     monkeypatch.setattr(pkg, "load_library", lambda: lib)
@@ -30,7 +33,10 @@ def _run(pkg, monkeypatch, call):
     monkeypatch.setattr(torch, "empty", empty_without_pinning)
     cpu = {"device": "cpu"}
     x, w, out = torch.zeros((4, 8), **cpu), torch.zeros((1, 8, 8), **cpu), torch.zeros((4, 8), **cpu)
-    pkg._call_device(pkg.OP_FORWARD, pkg.DType.BF16, pkg.DType.BF16, 8, 8, torch.tensor([4], **cpu), None, 4, x, w, out)
+    try:
+        pkg._call_device(pkg.OP_FORWARD, pkg.DType.BF16, pkg.DType.BF16, 8, 8, torch.tensor([4], **cpu), None, 4, x, w, out)
+    finally:
+        assert [t.device.type for t in pinned] == ["cpu"]
     return stream
 
 
@@ -53,3 +59,9 @@ def test_a_failing_call_waits_before_its_status_is_freed(pkg, monkeypatch, failu
     with pytest.raises(KeyboardInterrupt if failure == "interrupt" else pkg.GGError):
         _run(pkg, monkeypatch, call)
     assert stream[0].waits == 1
+
+
+def test_status_is_host_memory_whatever_the_default_device(pkg, monkeypatch):
+    with torch.device("meta"):
+        torch.empty(1)  # torch lists the functions that take a default device on first use: before the stand-ins
+        assert _run(pkg, monkeypatch, lambda *a: pkg.GG_OK).waits == 1

@@ -102,6 +102,15 @@ def test_bad_device_sizes_raise(pkg):
             pkg.grouped_gemm(a, w, lens)
 
 
+def test_default_device_is_the_gpu(pkg):
+    """A program may make the GPU torch's default device; the status of a device-size call stays host memory."""
+    a, w, _, _ = _inputs("fwd", "bf16", [5, 3], 64, 72)
+    want = pkg.grouped_gemm(a, w, [5, 3])
+    with torch.device(DEV):
+        for sizes in ([5, 3], torch.tensor([5, 3], dtype=torch.int64, device=DEV)):
+            assert torch.equal(pkg.grouped_gemm(a, w, sizes), want)
+
+
 def test_threads_and_streams(pkg, monkeypatch):
     """Four threads, each on a stream of its own with sizes of its own, 30 calls each."""
     monkeypatch.delenv("GG_SMALL", raising=False)
