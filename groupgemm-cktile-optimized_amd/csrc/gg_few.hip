@@ -105,27 +105,33 @@ __global__ void __launch_bounds__(W * 64) few_gemm_kernel(const KernelArgs args)
         // ---- the tile: group g, row tile tm, column tile tn (row tiles innermost, so that the
         // workgroups that share w rows run next to each other on one XCD) ----
         const int L = xcd_remap(t, total, grid, args.n_xcd);
-        int64_t   row0 = 0;
-        int       g = 0, gm = 0, local = 0;
-        for (int base = 0; base < args.group_num; base += 64) {
-            // the last group whose first tile is at most L (an empty group shares its successor's)
-            const bool live = base + lane < args.group_num;
-            if (args.d_lens == nullptr) {
-                const GroupEntry e = args.groups[live ? base + lane : 0];
-                lg.row0 = e.row0;
-                lg.m = e.m;
-                lg.tile0 = e.tile0;
+        // The group is the last one whose first tile is at most L (an empty group shares its successor's).
+        // A table of more than 64 groups is narrowed to 64 entries first, by 64 evenly spaced ones at a
+        // time: every load waits for the one before, and a scan in steps of 64 took a load per 64 groups
+        // for every tile (us per launch, scan -> this: 4096 groups of 8 rows, N = 128, K = 256 191 -> 54;
+        // the persistent kernel, which scans once per workgroup, 93).
+        int first = 0, span = args.group_num;
+        if (args.d_lens == nullptr) {
+            while (span > 64) {
+                const int      step = (span + 63) / 64;
+                const bool     live = lane * step < span;
+                const int      t0   = args.groups[live ? first + lane * step : first].tile0;
+                const uint64_t mask = __ballot(live && t0 <= L); // bit 0 is set: the range's first entry is at most L
+                const int      s    = 63 - __builtin_clzll(mask);
+                first += s * step;
+                span = min(step, span - s * step);
             }
-            const uint64_t mask = __ballot(live && lg.tile0 <= L);
-            if (mask == 0)
-                break;
-            const int s = 63 - __builtin_clzll(mask);
-            g           = base + s;
-            gm          = __builtin_amdgcn_readlane(lg.m, s);
-            local       = L - __builtin_amdgcn_readlane(lg.tile0, s);
-            row0 = static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(lg.row0), s))) |
-                   (static_cast<int64_t>(__builtin_amdgcn_readlane(static_cast<int>(lg.row0 >> 32), s)) << 32);
+            const GroupEntry e = args.groups[lane < span ? first + lane : first];
+            lg.row0  = e.row0;
+            lg.m     = e.m;
+            lg.tile0 = e.tile0;
         }
+        const int s     = 63 - __builtin_clzll(__ballot(lane < span && lg.tile0 <= L));
+        const int g     = first + s;
+        const int gm    = __builtin_amdgcn_readlane(lg.m, s);
+        const int local = L - __builtin_amdgcn_readlane(lg.tile0, s);
+        int64_t   row0  = static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(lg.row0), s))) |
+                       (static_cast<int64_t>(__builtin_amdgcn_readlane(static_cast<int>(lg.row0 >> 32), s)) << 32);
         const int mts = (gm + BM - 1) / BM;
         const int tn = local / mts, tm = local - tn * mts;
         row0 += static_cast<int64_t>(tm) * BM;

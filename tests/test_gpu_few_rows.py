@@ -140,6 +140,24 @@ def test_same_outputs_as_the_persistent_kernel(pkg, monkeypatch, op):
         assert torch.equal(o.view(torch.int16), outs[0].view(torch.int16))
 
 
+@pytest.mark.parametrize("b", [64, 65, 128, 129, 4096, 4097, 9000])
+@pytest.mark.parametrize("instance", [1, 3])
+def test_group_search(pkg, monkeypatch, b, instance):
+    """Tables of one, two and three levels of 64, whole and ragged, with empty groups at the start, at the end
+    and between: every row is multiplied with its own expert (integers: exact)."""
+    monkeypatch.delenv("GG_SMALL", raising=False)
+    monkeypatch.setenv("GG_FEW", str(instance))
+    gm = [0, 0] + [(7 * g * g + g // 64) % 5 for g in range(b - 5)] + [40, 0, 0]
+    rows = torch.repeat_interleave(torch.arange(b, device=DEV), torch.tensor(gm, device=DEV))
+    for device in (False, True):
+        print(f"[few search] {b} groups device={device}", flush=True)
+        c = Case(pkg, "fwd", "bf16", "bf16", gm, 24, 16, device, ints=True, seed=b).run()
+        assert "few-row" in c.plan.detail(), c.plan.detail()
+        ref = (c.a.float()[:, None, :] * c.b.float()[rows]).sum(-1)
+        assert torch.equal(c.out.float(), ref)
+        c.close()
+
+
 @pytest.mark.parametrize("b", [3, 70])
 def test_device_sizes_gaps_and_bad_groups(pkg, monkeypatch, b):
     """Rows outside every group stay as they were; a group whose rows do not fit is named and left
