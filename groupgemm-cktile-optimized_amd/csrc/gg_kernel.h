@@ -147,7 +147,7 @@ hipError_t launch_tail_reduce(const KernelArgs &args, bool fp16, int grid, hipSt
 // (int64 rows) and offs[group_num + 1] (int64 first rows) or null for back-to-back groups.
 // Groups outside [0, total_m) get no rows (forward / dgrad: no tiles) and are reported in the
 // header. out_rows > 0 (wgrad): every group owns ceil(out_rows / 256) * n_tiles tiles. One wave.
-// tile_m, n_tiles: the table's tiles. wide_n_tiles > 0: the header's total_tiles counts 256-row
+// tile_m (a power of two), n_tiles: the table's tiles. wide_n_tiles > 0: the header's total_tiles counts 256-row
 // tiles times it (a table of other tiles than 256 x 256, whose count goes to run_tiles).
 hipError_t launch_build_group_table(const int64_t *lens, const int64_t *offs, int group_num,
                                     int64_t total_m, int n_tiles, GroupEntry *table,
