@@ -586,18 +586,25 @@ constexpr double kOtherHbm16 = 6.8e6, kOtherHbm8 = 5.9e6;
 constexpr double kOtherFixedUs = 7.2, kOtherStepUs = 0.88;  // persistent kernel
 constexpr double kOtherSmallFixedUs = 1.8;                  // 128 x 128 tiles
 
-// Row tiles of bm rows: of the host's sizes, or of `rows` rows spread over the groups (device sizes:
-// a group whose average fills more than half a tile is expected to end in half a tile).
-double row_tiles(const int64_t *group_m, int group_num, int64_t rows, int bm) {
-    if (group_m == nullptr) {
-        const double avg = double(rows) / group_num;
-        return std::max(double(std::min<int64_t>(group_num, rows)), double(rows) / bm + (avg > bm / 2 ? 0.5 * group_num : 0.0));
+// Row tiles of 16, 32, .. 256 rows: of the host's sizes, or of `rows` rows spread over the groups (device
+// sizes: a group whose average fills more than half a tile is expected to end in half a tile). One pass
+// of shifts: a division per group and tile height took 0.4 ms of a plan's preparation for 32768 groups.
+struct RowTiles {
+    double tiles[5] = {};
+    RowTiles(const int64_t *group_m, int group_num, int64_t rows) {
+        int64_t sum[5] = {};
+        for (int g = 0; g < group_num && group_m != nullptr; ++g)
+            for (int i = 0; i < 5; ++i)
+                sum[i] += (group_m[g] + (16 << i) - 1) >> (4 + i);
+        for (int i = 0; i < 5; ++i) {
+            const double avg = double(rows) / group_num, bm = 16 << i;
+            tiles[i] = group_m != nullptr ? double(sum[i])
+                                          : std::max(double(std::min<int64_t>(group_num, rows)),
+                                                     double(rows) / bm + (avg > bm / 2 ? 0.5 * group_num : 0.0));
+        }
     }
-    double t = 0;
-    for (int g = 0; g < group_num; ++g)
-        t += static_cast<double>(gg::cdiv(group_m[g], bm));
-    return t;
-}
+    double of(int bm) const { return tiles[__builtin_ctz(static_cast<unsigned>(bm)) - 4]; }
+};
 
 // The few-row instance of a forward or dgrad plan (its problem set; group_m null: device sizes of
 // `rows` rows in all), or -1.
@@ -614,15 +621,16 @@ int choose_few_rows(const gg_plan *plan, const int64_t *group_m, int64_t rows, i
     const int64_t groups = std::min<int64_t>(plan->group_num, rows);
     const int64_t chunks = gg::cdiv(plan->k * es, 128); // 128 bytes of an operand row
     const double  bytes  = double(groups) * plan->n * plan->k * es + double(rows) * (plan->k * es + plan->n * 2);
+    const RowTiles row_tiles(group_m, plan->group_num, rows);
     // the plan that would run otherwise
-    const double tiles = row_tiles(group_m, plan->group_num, rows, gg::kTileM) * gg::cdiv(plan->n, gg::kTileN);
+    const double tiles = row_tiles.of(gg::kTileM) * gg::cdiv(plan->n, gg::kTileN);
     double       steps, fixed = kOtherFixedUs;
     if (group_m == nullptr || tiles > cus) {
         steps = std::max(1.0, std::ceil(tiles / cus)) * chunks * kOtherStepUs;
     } else {
         const int s = choose_splits(static_cast<int>(tiles), static_cast<int>(chunks), cus);
         steps       = gg::cdiv(chunks, s) * kOtherStepUs + (s > 1 ? kSplitUs + s * tiles * kSlabUs : 0.0);
-        const double units = row_tiles(group_m, plan->group_num, rows, gg::kSmallTile) * gg::cdiv(plan->n, gg::kSmallTile);
+        const double units = row_tiles.of(gg::kSmallTile) * gg::cdiv(plan->n, gg::kSmallTile);
         if (!f8 && !dgrad && small_tiles_win(static_cast<int64_t>(units), static_cast<int>(chunks), static_cast<int>(tiles), s,
                                              static_cast<int>(chunks), cus)) {
             if (forced < 0 && units > kFewMaxSmallTiles && rows > 64 * groups)
@@ -639,11 +647,11 @@ int choose_few_rows(const gg_plan *plan, const int64_t *group_m, int64_t rows, i
         const gg::FewInstance &f = gg::kFewInstances[i];
         // the kernel's tile index must not pass 2^31 (device sizes may put every row in each group)
         const int64_t nt   = gg::cdiv(plan->n, f.tile_n);
-        const double  most = group_m != nullptr ? row_tiles(group_m, plan->group_num, rows, f.tile_m)
+        const double  most = group_m != nullptr ? row_tiles.of(f.tile_m)
                                                 : double(plan->group_num) * double(gg::cdiv(rows, f.tile_m));
         if ((forced >= 0 && i != forced) || most * double(nt) > double(gg::kMaxLoopTiles))
             continue;
-        const double wgs    = row_tiles(group_m, plan->group_num, rows, f.tile_m) * nt;
+        const double wgs    = row_tiles.of(f.tile_m) * nt;
         const double staged = wgs * (f.tile_m + f.tile_n) * 128.0 * chunks;
         const double chain  = std::max(1.0, std::ceil(wgs / (cus * f.per_cu))) * (gg::cdiv(chunks, f.waves) * f.chunk_us + kFewRoundUs);
         const double us     = kFewFixedUs + std::hypot(bytes / kFewHbm, staged / stage, chain);
@@ -719,18 +727,18 @@ bool choose_wgrad_few(const gg_plan *plan, const int64_t *group_m, int64_t m_out
         return std::atoi(env) != 0;
     const bool f8      = plan->mode / 4 != gg::kIn16;
     const int  es      = f8 ? 1 : 2;
-    const auto average = [&](int rows_per, double least) { // K steps of a group
+    const auto average = [&](int rows_log2, int least) { // K steps of 2^rows_log2 rows of a group
         if (group_m == nullptr)
-            return std::max(least, double(rows) / plan->group_num / rows_per + 0.5);
-        double sum = 0;
+            return std::max<double>(least, std::ldexp(double(rows) / plan->group_num, -rows_log2) + 0.5);
+        int64_t sum = 0;
         for (int g = 0; g < plan->group_num; ++g)
-            sum += std::max(least, static_cast<double>(gg::cdiv(group_m[g], rows_per)));
-        return sum / plan->group_num;
+            sum += std::max<int64_t>(least, (group_m[g] + (1 << rows_log2) - 1) >> rows_log2);
+        return double(sum) / plan->group_num;
     };
     const double bytes  = double(plan->group_num) * m_out * plan->n * 2 + double(rows) * (m_out + plan->n) * es;
     const double wide   = double(plan->group_num) * gg::cdiv(m_out, gg::kTileM) * gg::cdiv(plan->n, gg::kTileN);
-    const double steps  = average(f8 ? 128 : 64, gg::kCrossMinStepsHost);
-    const double chunks = average(f8 ? 128 : 32, 0.0);
+    const double steps  = average(f8 ? 7 : 6, gg::kCrossMinStepsHost);
+    const double chunks = average(f8 ? 7 : 5, 0);
     const double per_cu = std::max(0.25, tiles / cus);
     const double other  = kWgradFixedUs + std::hypot(bytes / kWgradHbm, std::ceil(wide / cus) *
                                                                            (f8 ? 1.75 + 1.2 * steps : 2.1 + 1.14 * steps));
