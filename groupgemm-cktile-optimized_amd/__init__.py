@@ -386,7 +386,7 @@ def _call_host(op: int, a_dtype: DType, b_dtype: DType, n: int, k: int, group_m:
     lib, count = load_library(), len(group_m)
     stream = torch.cuda.current_stream(a.device)
     gm = (ctypes.c_int64 * max(1, count))(*group_m)
-    need = ctypes.c_size_t(4096 + 16 * count)  # the tables of any plan without partial sums or small tiles
+    need = ctypes.c_size_t(max(1 << 20, 96 * count))  # the tables of a plan without partial sums
     sa, sb = (0, 0) if a_scale is None else (a_scale.data_ptr(), b_scale.data_ptr())
     for _ in range(2):
         ws = torch.empty(need.value, dtype=torch.uint8, device=a.device)

@@ -41,7 +41,7 @@ struct gg_plan {
     std::vector<gg::SmallTile>  small_list;
     size_t                      ws_bytes = 0;
     void                       *mem      = nullptr;
-    bool                        one_call = false; // gg_call: no descriptors, no detail text
+    bool                        one_call = false; // gg_call: no detail text, descriptors where one_call_desc
     gg::GroupEntry     *d_groups    = nullptr;
     gg::KernelArgs      args{};
     std::string         detail;
@@ -791,6 +791,17 @@ int use_few_rows(gg_plan *plan, const int64_t *group_m, const float *x_scale, co
     return GG_OK;
 }
 
+// Whether a gg_call plan, which is used once, has tile descriptors (setup_tile_desc): where the walk
+// without them is long for the tiles there are. A workgroup's scan of the table takes about 90 ns per
+// group, a descriptor about 20-40 ns to build and bring to the device. Torch-level forward calls, us
+// without -> with descriptors (MI355X): 2048 groups of 8 rows, N = K = 256, 2048 tiles 434 -> 238; 256
+// groups, 512 x 512, 512 tiles 90 -> 77; 128 groups, 1024 x 512, 512 tiles 77 -> 71. Without it stays
+// better for 1024 groups and 8192 tiles (490, with: 501), 64 groups, 2048 x 1024, 512 tiles (91, 94), 32
+// of 520 rows, 2880 x 2880 (279, 296) and 8 of 4096, 14336 x 4096 (2596, 2625).
+bool one_call_desc(const gg_plan *plan) {
+    return plan->group_num >= 128 && plan->total_tiles <= 4 * int64_t(plan->group_num);
+}
+
 // Tile descriptors of forward, dgrad and wgrad plans of whole tiles (host-size tables): every
 // workgroup's tiles in the kernel's own walk (xcd_remap, then locate_tile over the plan's group
 // table with its tile rows and N-tiles), so that the kernel reads a tile's first row, group and
@@ -801,8 +812,8 @@ int use_few_rows(gg_plan *plan, const int64_t *group_m, const float *x_scale, co
 int setup_tile_desc(gg_plan *plan, const int64_t *group_m) {
     gg::KernelArgs &a   = plan->args;
     const char     *env = std::getenv("GG_TILE_DESC");
-    if ((env != nullptr && env[0] == '0') || plan->one_call || a.splits > 1 || a.tail_splits > 1 || plan->grid <= 0 ||
-        !gg::desc_rows_fit(group_m, plan->group_num, plan->total_m))
+    if ((env != nullptr && env[0] == '0') || (plan->one_call && !one_call_desc(plan)) || a.splits > 1 ||
+        a.tail_splits > 1 || plan->grid <= 0 || !gg::desc_rows_fit(group_m, plan->group_num, plan->total_m))
         return GG_OK;
     const int per_wg = static_cast<int>(gg::cdiv(plan->total_tiles, plan->grid));
     if (per_wg > gg::kMaxDescPerWg)

@@ -69,6 +69,32 @@ def test_calls_give_the_bits_of_plans(pkg, monkeypatch, case, small):
         assert torch.equal(one.view(torch.int16), plan.view(torch.int16))
 
 
+# more groups than fill one launch of the table upload (3584 bytes of kernel arguments) and its limit of 32
+# KB, with and without tile descriptors in the call's plan (from 128 groups on, up to 4 tiles per group)
+MANY = [
+    ("fwd", "bf16", 127, 40, 24), ("fwd", "bf16", 300, 512, 64), ("fwd", "fp16", 300, 1032, 64), ("fwd", "bf16", 2100, 24, 40),
+    ("fwd", "bf16", 9000, 16, 16), ("fwd", "e4m3", 300, 520, 48), ("dgrad", "bf16", 300, 40, 512), ("dgrad", "bf16", 2100, 40, 16),
+    ("wgrad", "bf16", 300, 24, 40), ("wgrad", "fp16", 2100, 16, 24),
+]
+
+
+@pytest.mark.parametrize("small", ["0", None])
+@pytest.mark.parametrize("case", range(len(MANY)))
+def test_many_groups(pkg, monkeypatch, case, small):
+    """Rows are ragged, some groups empty; the plan route gives the same bits."""
+    if small is None:
+        monkeypatch.delenv("GG_SMALL", raising=False)
+    op, t, b, n, k = MANY[case]
+    gm = [(7 * g * g + g // 64) % 5 for g in range(b - 1)] + [300]
+    a, other, sa, sb = _inputs(op, t, gm, n, k, seed=case)
+    print(f"[call] {op} {t} {b} groups N={n} K={k}", flush=True)
+    one = _call(pkg, op, t, a, other, gm, sa, sb)
+    plan = _call(pkg, op, t, a, other, gm, sa, sb, stream=_stream())
+    torch.cuda.synchronize(DEV)
+    assert not torch.isnan(one.float()).any() and one.float().abs().max() > 1
+    assert torch.equal(one.view(torch.int16), plan.view(torch.int16))
+
+
 def test_workspace_protocol(pkg, monkeypatch):
     """Too little workspace enqueues nothing and says how much is needed; that much is enough."""
     monkeypatch.setenv("GG_SPLIT_K", "3")
