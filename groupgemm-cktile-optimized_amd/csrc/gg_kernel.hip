@@ -369,8 +369,14 @@ hipError_t launch_upload(void *dst, const void *src, size_t bytes, hipStream_t s
     if (bytes % 16 != 0 || (reinterpret_cast<uintptr_t>(dst) & 15u) != 0)
         return hipErrorInvalidValue;
     if (bytes > kUploadMaxBytes) {
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
-        return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        hipError_t             e       = hipStreamIsCapturing(stream, &capture);
+        if (e == hipSuccess && capture == hipStreamCaptureStatusNone) {
+            e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
+            return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+        }
+        if (e != hipSuccess)
+            return e;
     }
     // 3.5 KB of arguments at most per launch (64 groups' table is 1 KB)
     for (size_t at = 0; at < bytes;) {

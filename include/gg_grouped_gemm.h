@@ -231,12 +231,15 @@ int gg_run_device_lens_noalloc(int op, int a_dtype, int b_dtype, int group_num, 
 
 /*
  * A prepare, run and release of host-size groups in one call on `stream`, in the caller's device
- * memory: nothing is allocated, freed or waited for. op, a, b, out and the scales as in
+ * memory: nothing is allocated or freed there. Nothing is waited for either, unless the call's tables
+ * are larger than 32 KB (from about 400 groups on): then the call waits for the stream while they
+ * are copied, except while it is captured into a graph. op, a, b, out and the scales as in
  * gg_prepare_device_lens_op, group_m and the requirements as in the matching host-size prepare
  * (gg_prepare, gg_prepare_fp8, gg_prepare_dgrad, ...). workspace: workspace_bytes of 256-byte
  * aligned device memory that must stay valid until the work on `stream` is done; if that is too
  * little, GG_ERR_WORKSPACE comes back with the size in *needed and nothing is enqueued. (Group tables
- * take 16 bytes per group; split-K partial sums up to 64 MB.) No counterpart in the reference.
+ * take 16 bytes per group, for 128 groups and more up to 80; split-K partial sums up to 64 MB.) No
+ * counterpart in the reference.
  */
 int gg_call(int op, int a_dtype, int b_dtype, int group_num, int64_t n, int64_t k, const int64_t *group_m,
             const void *a, const void *b, const float *a_scale, const float *b_scale, void *out,

@@ -95,6 +95,38 @@ def test_many_groups(pkg, monkeypatch, case, small):
     assert torch.equal(one.view(torch.int16), plan.view(torch.int16))
 
 
+@pytest.mark.parametrize("b", [40, 300, 3000])
+def test_call_replays_in_a_graph(pkg, monkeypatch, b):
+    """gg_call captured with tables of one launch, of several and past the size that is copied outside a
+    capture: nothing is waited for, and every replay, with eager work between, writes the tables again and
+    gives the plan's bits."""
+    monkeypatch.delenv("GG_SMALL", raising=False)
+    gm = [(7 * g * g) % 5 for g in range(b - 1)] + [300]
+    a, w, _, _ = _inputs("fwd", "bf16", gm, 72, 40, seed=b)
+    want = pkg.grouped_gemm(a, w, gm, stream=_stream())
+    lib, need, out = pkg.load_library(), ctypes.c_size_t(0), torch.empty_like(want)
+    sizes, ws = (ctypes.c_int64 * b)(*gm), torch.empty(1 << 20, dtype=torch.uint8, device=DEV)
+
+    def call():
+        st = lib.gg_call(pkg.OP_FORWARD, 0, 0, b, 72, 40, sizes, a.data_ptr(), w.data_ptr(), 0, 0, out.data_ptr(),
+                         ws.data_ptr(), ws.numel(), ctypes.byref(need), torch.cuda.current_stream(DEV).cuda_stream)
+        assert st == pkg.GG_OK, pkg.last_error()
+
+    call()
+    torch.cuda.synchronize(DEV)
+    assert torch.equal(out, want) and (need.value > 32768) == (b == 3000)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for replay in range(3):
+        out.fill_(float("nan"))
+        ws.zero_()
+        pkg.grouped_gemm(a, w, gm)
+        graph.replay()
+        torch.cuda.synchronize(DEV)
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)), replay
+
+
 def test_workspace_protocol(pkg, monkeypatch):
     """Too little workspace enqueues nothing and says how much is needed; that much is enough."""
     monkeypatch.setenv("GG_SPLIT_K", "3")
