@@ -563,23 +563,24 @@ int allocate_plan(gg_plan *p, hipStream_t s) {
 // whose groups have few rows or whose whole problem is small: there the 256 x 256 tiles of the
 // persistent kernel (and the 128 x 128 ones) leave CUs idle or run one long chain of K steps each.
 // Chosen by a launch-time model in microseconds, the lesser instance's time against the plan
-// that would run otherwise, taken at kFewGain of it. Both sides add the parts' squares (the memory
+// that would run otherwise, taken at a share of it (few_gain). Both sides add the parts' squares (the memory
 // traffic, the operands' way into LDS and the chain of K steps overlap, but not fully):
 //   few:   kFewFixedUs + |HBM bytes / kFewHbm, staged bytes / kFewStage, rounds of workgroups x
 //          (chunks per wave x chunk_us + kFewRoundUs)|
 //   other: fixed + |HBM bytes / kOtherHbm, K steps of the busiest workgroup|
 // Fitted to 300 random forward and dgrad problems of 1-64 groups, 1-1000 rows each, N and K
-// 512-14336, bf16 and fp8 (MI355X, each instance and the other plan timed): the choice gives
-// 1.70x over the other plans in the geometric mean (the best instance of each 1.76x) and a loss on
-// none. Examples (us, other -> few): 4 x 256 rows, 512 x 1024 12.3 -> 5.4;
-// 3 x 5 rows, 3328 x 12256 199 -> 56; 3 x 14 rows dgrad, 1208 x 2048 25.6 -> 6.3; 16 x 64 rows,
-// 2048 x 1408 29.5 -> 22.5; left: 8 x 128 rows, 4096 x 7168 100 (few 131). With rows for whole
+// 512-14336, bf16 and fp8 (MI355X, each instance and the other plan timed). On 1900 others, 40 % of them
+// with contractions over 6000, each with its operands in cache and from HBM in turn, the choice gives
+// 1.71x (HBM: 1.58x) over the other plans in the geometric mean, the best of each 1.82x (1.66x), and is
+// slower in cache or from HBM on 16 of them (0.71-0.97x). Examples (us, other -> few): 4 x 256 rows,
+// 512 x 1024 12.3 -> 6.4; 3 x 5 rows (device sizes), 3328 x 12256 130 -> 38; 3 x 14 rows dgrad, 1208 x 2048
+// 25.3 -> 6.0; 36 x 16 rows, 2048 x 1024 35.9 -> 23.4; left: 8 x 128 rows, 4096 x 7168 100 (few 131). With rows for whole
 // tiles, the staged bytes (each small tile stages its own operands) decide against it.
 // Plans of more than kFewMaxSmallTiles 128 x 128 tiles whose groups average over 64 rows keep them:
 // the few-row tiles ran 0.73-1.28x there (7 of the 300 problems), and the model is no better than that.
 // GG_SMALL in the environment (0: no small tiles, 1: 128 x 128 tiles) turns it off; without it,
 // GG_FEW=<i> takes instance i (GG_FEW=-1: none).
-constexpr double kFewGain = 0.85, kFewFixedUs = 1.6, kFewRoundUs = 1.9;
+constexpr double kFewFixedUs = 1.6, kFewRoundUs = 1.9;
 constexpr double kFewHbm = 6.2e6, kFewStageFwd = 22e6, kFewStageDgrad16 = 15e6, kFewStageDgrad8 = 10.5e6; // bytes per us
 constexpr int    kFewMaxSmallTiles = 64;
 constexpr double kOtherHbm16 = 6.8e6, kOtherHbm8 = 5.9e6;
@@ -605,6 +606,16 @@ struct RowTiles {
     }
     double of(int bm) const { return tiles[__builtin_ctz(static_cast<unsigned>(bm)) - 4]; }
 };
+
+// The share of the other plan's time that a few-row plan must promise. Where the contraction is long, most
+// of the time is w's way from HBM and the model, fitted with w in the caches, promises too much: with
+// 0.85 throughout, 69 of the 1900 problems were slower than the other plan, down to 0.63x, nearly all with
+// less than 1.4 rounds of workgroups. dgrad with less than 3/4 of a round reads w's rows in pieces of 32-128
+// bytes and has the most of them (2 x 57 rows forward, 5632 x 13008 87 -> 120 us; 3 x 26 dgrad, 1024 x 13888
+// 40 -> 63).
+double few_gain(bool dgrad, int64_t chunks, double rounds) {
+    return chunks < 64 || rounds >= 1.4 ? 0.85 : dgrad && rounds < 0.75 ? 0.53 : 0.61;
+}
 
 // The few-row instance of a forward or dgrad plan (its problem set; group_m null: device sizes of
 // `rows` rows in all), or -1.
@@ -642,7 +653,7 @@ int choose_few_rows(const gg_plan *plan, const int64_t *group_m, int64_t rows, i
     const double other = fixed + std::hypot(bytes / (f8 ? kOtherHbm8 : kOtherHbm16), steps);
     const double stage = !dgrad ? kFewStageFwd : f8 ? kFewStageDgrad8 : kFewStageDgrad16;
     int          best  = -1;
-    double       least = kFewGain * other;
+    double       least = 0, rounds = 0;
     for (int i = 0; i < gg::kFewInstanceCount; ++i) {
         const gg::FewInstance &f = gg::kFewInstances[i];
         // the kernel's tile index must not pass 2^31 (device sizes may put every row in each group)
@@ -653,14 +664,16 @@ int choose_few_rows(const gg_plan *plan, const int64_t *group_m, int64_t rows, i
             continue;
         const double wgs    = row_tiles.of(f.tile_m) * nt;
         const double staged = wgs * (f.tile_m + f.tile_n) * 128.0 * chunks;
-        const double chain  = std::max(1.0, std::ceil(wgs / (cus * f.per_cu))) * (gg::cdiv(chunks, f.waves) * f.chunk_us + kFewRoundUs);
+        const double round  = wgs / (cus * f.per_cu);
+        const double chain  = std::max(1.0, std::ceil(round)) * (gg::cdiv(chunks, f.waves) * f.chunk_us + kFewRoundUs);
         const double us     = kFewFixedUs + std::hypot(bytes / kFewHbm, staged / stage, chain);
-        if (forced >= 0 || us < least) {
-            least = us;
-            best  = i;
+        if (best < 0 || us < least) {
+            least  = us;
+            best   = i;
+            rounds = round;
         }
     }
-    return best;
+    return forced >= 0 || least < few_gain(dgrad, chunks, rounds) * other ? best : -1;
 }
 
 // The few-row kernel's operand format of a plan.

@@ -25,13 +25,13 @@
 // row and column (N % 8 == 0: four columns are all valid or not).
 //
 // Measured (MI355X, us per launch back to back, the plans that ran before -> this kernel): bf16
-// forward 4 x 256 rows, 512 x 1024 12.3 -> 5.4; 36 x 16, 2048 x 1024 43.1 -> 29.1 (5.3 TB/s of w);
-// 16 x 64, 2048 x 1408 29.5 -> 22.5; 1 x 512, 2880 x 2880 28.8 -> 19.7; 3 x 5 (device sizes), 3328 x
-// 12256 199 -> 56; fp8 forward 4 x 3, 9840 x 800 15.1 -> 9.1; dgrad bf16 3 x 14, 1208 x 2048 25.6 ->
-// 6.3, fp8 32 x 64, 2512 x 768 28.0 -> 17.8. The ring's depth and the waves were swept (29
+// forward 4 x 256 rows, 512 x 1024 12.3 -> 6.4; 36 x 16, 2048 x 1024 35.9 -> 23.4 (6.4 TB/s of w, part of
+// it from the Infinity Cache); 1 x 512, 2880 x 2880 28.5 -> 20.3; 3 x 5 (device sizes), 3328 x 12256 130 -> 38;
+// fp8 forward 4 x 3, 9840 x 800 14.7 -> 6.0; dgrad bf16 3 x 14, 1208 x 2048 25.3 ->
+// 6.0, fp8 32 x 64, 2512 x 768 26.4 -> 17.3. The ring's depth and the waves were swept (29
 // combinations of 1-8 row blocks, 1-4 column blocks, 1-16 waves, 1-4 chunks): what pays is many
-// small workgroups per CU, not a deep ring (16 rows: 4 waves x 2 chunks, 2 per CU, 29.1 on the second
-// shape; x 4 chunks, 1 per CU, 34.8). More rows per tile than 64 lose to the 128 x 128 tiles: every
+// small workgroups per CU, not a deep ring (16 rows: 4 waves x 2 chunks, 2 per CU, 29.1 against
+// 34.8 with 4 chunks, 1 per CU, on the second shape, w from HBM). More rows per tile than 64 lose to the 128 x 128 tiles: every
 // tile stages its own operands, about 15-22 TB/s over the chip.
 #include "gg_few.h"
 #include "gg_kernel_impl.h"

@@ -240,3 +240,26 @@ def test_planner_choice(pkg, monkeypatch, case):
         c = Case(pkg, op, t, t, gm, n, k, device, ints=True)
         assert ("few-row" in c.plan.detail()) == few, c.plan.detail()
         c.close()
+
+
+# long contractions (rows of 8 KB and more) in less than 1.4 rounds of workgroups promise less than the model
+# says: (op, group rows, N, K, few-row tiles expected)
+LONG = [
+    ("dgrad", [26] * 3, 13888, 1024, False),   # 0.19 rounds, predicted at 0.73 of the persistent plan
+    ("fwd", [16] * 2, 512, 12288, True),       # 0.03 rounds, far below it
+    ("fwd", [12] * 12, 4096, 4160, True),      # 1.5 rounds: the usual share
+]
+
+
+@pytest.mark.parametrize("case", range(len(LONG)))
+def test_planner_choice_for_long_contractions(pkg, monkeypatch, case):
+    monkeypatch.delenv("GG_SMALL", raising=False)
+    op, gm, n, k, few = LONG[case]
+    p = torch.empty(16, dtype=torch.uint8, device=DEV).data_ptr()  # plans read no operand
+    if op == "dgrad":
+        plan = pkg.BackwardPlan("dgrad", pkg.DType.BF16, n, k, gm, p, p, p, _stream())
+    else:
+        plan = pkg.make_mi355x_backend()
+        assert plan.prepare(pkg.GroupedGemmProblem(pkg.DType.BF16, len(gm), n, k, gm, p, p, p), _stream()) == ""
+    assert ("few-row" in plan.detail()) == few, plan.detail()
+    plan.release()
