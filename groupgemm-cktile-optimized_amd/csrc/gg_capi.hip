@@ -712,18 +712,19 @@ std::string few_detail(const gg_plan *plan, const std::string &what) {
 // 128 x 128 tiles (gg_wfew.hip) for wgrad plans whose groups have few rows: the persistent kernel
 // runs at least four K steps per 256 x 256 tile and stores it 8 bytes per lane and row, this one
 // runs the chunks there are and stores whole rows. Chosen by a launch-time model in microseconds,
-// taken at kWgradFewGain of the persistent plan's time (|a, b| = sqrt(a^2 + b^2)):
+// taken at a share (gain) of the persistent plan's time (|a, b| = sqrt(a^2 + b^2)):
 //   few:        kWgradFewFixedUs + |bytes / kWgradFewHbm,
 //                                   tiles per CU x tile + chunks x |one chunk's latency, tiles per CU x chunk||
 //   persistent: kWgradFixedUs + |bytes / kWgradHbm, rounds x (tile + max(4, K steps) x step)|
 // with the groups' average K steps. Fitted to 320 random problems of 1-64 groups, 1-8000 rows each,
-// n and k 512-14336, bf16 and fp8 (MI355X, both kernels timed): the choice gives 1.41x over the
-// persistent kernel in the geometric mean, 0.95-0.99x on three problems and no loss elsewhere. Up to
-// 64 rows per group 1.8x, 65-256 1.5x; above 500 rows it pays where 256 x 256 tiles leave CUs idle (1.3x)
-// and loses elsewhere (0.7-0.9x: a 64 x 64 quarter per wave reads twice the LDS bytes per MFMA of the
-// persistent kernel's 128 x 128).
+// n and k 512-14336, bf16 and fp8 (MI355X, both kernels timed). On 900 others that the model takes at 0.9,
+// half of them of 300-3500 rows per group, each with its operands in cache and from HBM in turn: up to
+// 64 rows per group 1.8x (HBM 1.8x), 65-256 1.5x. Past 300 rows it pays where 256 x 256 tiles leave CUs idle,
+// but inputs from HBM cost it more than the persistent kernel, and of the problems under two rounds of
+// workgroups 41 were slower, down to 0.71x; at 0.73 two are (0.94x). With CUs full it loses (0.7-0.9x: a 64 x 64
+// quarter per wave reads twice the LDS bytes per MFMA of the persistent kernel's 128 x 128).
 // GG_SMALL in the environment turns it off; without it, GG_WFEW=1 takes it and GG_WFEW=0 does not.
-constexpr double kWgradFewGain = 0.9, kWgradFewFixedUs = 3.7, kWgradFixedUs = 7.8; // us
+constexpr double kWgradFewFixedUs = 3.7, kWgradFixedUs = 7.8; // us
 constexpr double kWgradFewHbm = 6.1e6, kWgradHbm = 5.1e6;                          // bytes per us
 
 int64_t wgrad_few_tiles(const gg_plan *plan, int64_t m_out) {
@@ -758,7 +759,8 @@ bool choose_wgrad_few(const gg_plan *plan, const int64_t *group_m, int64_t m_out
     const double few    = kWgradFewFixedUs +
                        std::hypot(bytes / kWgradFewHbm, f8 ? 0.05 * per_cu + chunks * std::hypot(0.98, 0.55 * per_cu)
                                                            : 0.32 * per_cu + chunks * std::hypot(0.43, 0.24 * per_cu));
-    return few < kWgradFewGain * other;
+    const double gain = rows > 300 * int64_t(plan->group_num) && tiles < 8 * cus ? 0.73 : 0.9; // (4 per CU)
+    return few < gain * other;
 }
 
 // The launch of such a plan, one workgroup per tile in whole XCD rows (after fill_args; m_out: the

@@ -187,3 +187,22 @@ def test_more_tiles_than_one_launch_takes(pkg, monkeypatch):
     torch.cuda.synchronize(DEV)
     lib.gg_release(plan)
     assert torch.count_nonzero(out) == 0
+
+
+# past 300 rows per group the share it must promise is smaller in less than two rounds of workgroups:
+# (group rows, N, K, few-row tiles expected)
+PAST_300 = [
+    ([1193] * 5, 6432, 512, False),    # 1.0 rounds, predicted at 0.79 of the persistent plan
+    ([316] * 11, 5376, 3344, True),    # 12 rounds, 0.89
+    ([320] * 4, 512, 512, True),       # 0.06 rounds, far below it
+]
+
+
+@pytest.mark.parametrize("case", range(len(PAST_300)))
+def test_planner_choice_past_300_rows(pkg, monkeypatch, case):
+    monkeypatch.delenv("GG_SMALL", raising=False)
+    gm, n, k, few = PAST_300[case]
+    p, e4 = torch.empty(16, dtype=torch.uint8, device=DEV).data_ptr(), _gdt(pkg, "e4m3")  # plans read no operand
+    plan = pkg.BackwardPlan("wgrad", e4, n, k, gm, p, p, p, _stream(), other_dtype=e4, grad_scale=p, other_scale=p)
+    assert ("few-row" in plan.detail()) == few, plan.detail()
+    plan.release()
