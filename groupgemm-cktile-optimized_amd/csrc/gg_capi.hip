@@ -1122,7 +1122,9 @@ int plan_device_lens(gg_plan *plan, TableMemory memory, void *given, int op, int
 }
 
 int run_few(const gg_plan *plan, hipStream_t s) {
-    const hipError_t e = plan->wgrad_few ? gg::launch_wgrad_few(plan->args, few_format(plan), plan->grid, s) : gg::launch_few_gemm(plan->args, few_format(plan), plan->mode % 4 == gg::kDgrad, plan->few, plan->grid, s);
+    const hipError_t e = plan->wgrad_few ? gg::launch_wgrad_few(plan->args, few_format(plan), plan->grid, s)
+                                         : gg::launch_few_gemm(plan->args, few_format(plan), plan->mode % 4 == gg::kDgrad,
+                                                               plan->few, plan->grid, s);
     return e == hipSuccess ? GG_OK : hip_fail(e, "few-row GEMM launch");
 }
 

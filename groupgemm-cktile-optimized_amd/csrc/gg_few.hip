@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(W * 64) few_gemm_kernel(const KernelArgs args)
     constexpr int kSums = W * BM * kSumStride * 4;
     constexpr int kLds = kSums > kRing ? kSums : kRing;
     static_assert(kLds <= 160 * 1024, "LDS");
-    static_assert((S - 1) * kDma <= 63, "vmcnt");
+    static_assert(S >= 1 && S <= 2 && (S - 1) * kDma <= 63, "vmcnt: one chunk behind the current one at most");
     __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -195,10 +195,6 @@ __global__ void __launch_bounds__(W * 64) few_gemm_kernel(const KernelArgs args)
             const int left = mine - 1 - c; // chunks of this wave still behind c, at most S - 1 in flight
             if (left >= S - 1)
                 wait_vm<(S - 1) * kDma>();
-            else if (S > 2 && left == 1)
-                wait_vm<kDma>();
-            else if (S > 3 && left == 2)
-                wait_vm<(S > 3 ? 2 : 0) * kDma>();
             else
                 wait_vm<0>();
             const unsigned char *sa = lds + wave * (S * kChunk) + stage * kChunk, *sb = sa + kARegion;

@@ -34,16 +34,17 @@ typedef __attribute__((address_space(3))) i32x2   lds_wi32x2;
 constexpr int kWT = kWgradFewTile; // 128 x 128 outputs per workgroup
 constexpr int kWRow = 272;         // staged output row stride (256 bytes + 16)
 
-template <int FMT, int R, int S, int OCC>
-__global__ void __launch_bounds__(kWgradFewThreads, OCC) wgrad_few_kernel(const KernelArgs args) {
+template <int FMT>
+__global__ void __launch_bounds__(kWgradFewThreads, 4) wgrad_few_kernel(const KernelArgs args) {
     constexpr bool kF8   = FMT >= kFewE4M3;
     constexpr bool kF16  = FMT == kFewF16;
     constexpr int  es    = kF8 ? 1 : 2;
-    constexpr int  kc    = R;                // rows per chunk
+    constexpr int  kc    = kF8 ? 128 : 32;   // rows per chunk
+    constexpr int  S     = kF8 ? 1 : 2;      // chunks in the ring
     constexpr int  row_b = kWT * es;         // bytes of a staged row
     constexpr int  pieces = row_b / 16;      // per row: 16 or 8
     constexpr int  rows_dma = 64 / pieces;   // rows per DMA: 4 or 8
-    constexpr int  kOp = R * row_b, kD = kOp / 4096; // bytes of an operand's chunk, DMAs per wave
+    constexpr int  kOp = kc * row_b, kD = kOp / 4096; // bytes of an operand's chunk, DMAs per wave
     __shared__ __attribute__((aligned(1024))) unsigned char lds[kWT * kWRow > 2 * S * kOp ? kWT * kWRow : 2 * S * kOp];
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int N = args.n, MO = args.m_out;
@@ -111,9 +112,8 @@ __global__ void __launch_bounds__(kWgradFewThreads, OCC) wgrad_few_kernel(const 
             acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int wm = wave >> 1, wn = wave & 1, fr = lane & 15, fq = lane >> 4;
     const int chunks = (m + kc - 1) / kc;
-    if constexpr (S > 1)
-        for (int c = 0; c < min(S - 1, chunks); ++c)
-            issue(c);
+    if (S == 2 && chunks > 0)
+        issue(0);
     for (int c = 0; c < chunks; ++c) {
         if constexpr (S == 1) {
             if (c > 0)
@@ -121,12 +121,9 @@ __global__ void __launch_bounds__(kWgradFewThreads, OCC) wgrad_few_kernel(const 
             issue(c);
             wait_vm_lds_barrier<0>();
         } else {
-            if (c + S - 2 < chunks)
-                wait_vm_lds_barrier<(S - 2) * 2 * kD>();
-            else
-                wait_vm_lds_barrier<0>();
-            if (c + S - 1 < chunks)
-                issue(c + S - 1);
+            wait_vm_lds_barrier<0>(); // chunk c has landed and chunk c - 1 is read
+            if (c + 1 < chunks)
+                issue(c + 1);
         }
         const unsigned char *sc = lds + (c % S) * (2 * kOp);
         if constexpr (kF8) {
@@ -155,38 +152,35 @@ __global__ void __launch_bounds__(kWgradFewThreads, OCC) wgrad_few_kernel(const 
                         fb[j], fa, acc[i][j], FMT == kFewE5M2 ? 1 : 0, FMT == kFewE4M3 ? 0 : 1, 0, 0, 0, 0);
             }
         } else {
+            auto frag = [&](int op, int blk) { // 16 columns from 16 blk, 32 rows
+                i32x4 v;
 #pragma unroll
-            for (int kh = 0; kh < R / 32; ++kh) {
-                auto frag = [&](int op, int blk) { // 16 columns from 16 blk, rows 32 kh .. + 31
-                    i32x4 v;
+                for (int h = 0; h < 2; ++h) {
+                    const int   row = 8 * fq + 4 * h + (fr >> 2);
+                    const i32x2 t = __builtin_bit_cast(
+                        i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                   (lds_wtr16 *)(sc + op * kOp + row * row_b + (((2 * blk + ((fr & 3) >> 1)) ^ swz(row)) << 4) +
+                                                 (fr & 1) * 8)));
+                    v[2 * h]     = t[0];
+                    v[2 * h + 1] = t[1];
+                }
+                return v;
+            };
+            i32x4 fb[4];
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const int   row = 32 * kh + 8 * fq + 4 * h + (fr >> 2);
-                        const i32x2 t = __builtin_bit_cast(
-                            i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                       (lds_wtr16 *)(sc + op * kOp + row * row_b + (((2 * blk + ((fr & 3) >> 1)) ^ swz(row)) << 4) +
-                                                     (fr & 1) * 8)));
-                        v[2 * h]     = t[0];
-                        v[2 * h + 1] = t[1];
-                    }
-                    return v;
-                };
-                i32x4 fb[4];
+            for (int j = 0; j < 4; ++j)
+                fb[j] = frag(1, wn * 4 + j);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const i32x4 fa = frag(0, wm * 4 + i);
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    fb[j] = frag(1, wn * 4 + j);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const i32x4 fa = frag(0, wm * 4 + i);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if constexpr (kF16)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(wf16x8, fb[j]),
-                                                                               __builtin_bit_cast(wf16x8, fa), acc[i][j], 0, 0, 0);
-                        else
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(wbf16x8, fb[j]),
-                                                                                __builtin_bit_cast(wbf16x8, fa), acc[i][j], 0, 0, 0);
-                }
+                    if constexpr (kF16)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(wf16x8, fb[j]),
+                                                                           __builtin_bit_cast(wf16x8, fa), acc[i][j], 0, 0, 0);
+                    else
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(wbf16x8, fb[j]),
+                                                                            __builtin_bit_cast(wbf16x8, fa), acc[i][j], 0, 0, 0);
             }
         }
     }
@@ -216,9 +210,7 @@ __global__ void __launch_bounds__(kWgradFewThreads, OCC) wgrad_few_kernel(const 
 } // namespace
 
 template <int FMT> void launch_format(const KernelArgs &a, int grid, hipStream_t s) {
-    constexpr bool f8 = FMT >= kFewE4M3;
-    hipLaunchKernelGGL((wgrad_few_kernel<FMT, f8 ? 128 : 32, f8 ? 1 : 2, 4>), dim3(static_cast<unsigned>(grid)),
-                       dim3(kWgradFewThreads), 0, s, a);
+    hipLaunchKernelGGL(wgrad_few_kernel<FMT>, dim3(static_cast<unsigned>(grid)), dim3(kWgradFewThreads), 0, s, a);
 }
 
 hipError_t launch_wgrad_few(const KernelArgs &a, int format, int grid, hipStream_t s) {

@@ -78,7 +78,8 @@ SHAPES = [
     ([31, 0, 32, 33, 1, 129], 144, 272),
     ([127, 128, 257], 128, 16),
     ([3, 0] * 35, 32, 144),  # 70 groups (device sizes: the table kernel)
-    ([700, 5], 1040, 656),   # more than one round of tiles per XCD run
+    ([700, 5], 1040, 656),   # partial tiles in both widths
+    ([9, 0, 40, 33] * 5, 1040, 1040),  # 1620 tiles: a whole round of 1024 in the XCD remap and a partial one
 ]
 
 
