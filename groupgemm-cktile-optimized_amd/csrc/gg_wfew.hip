@@ -6,7 +6,9 @@
 // and multiply. A chunk of the group's rows (32, in a ring of two; fp8: 128, one) goes from global
 // memory to LDS by DMA in row order (4 consecutive lanes on 64 contiguous bytes: 16 cycles per KB
 // of the address unit) and is read transposed (ds_read_b64_tr_b16 / _b8) for both operands. Row r's
-// 16-byte piece p sits at p ^ swz(r), which spreads the rows that one read pass covers over the banks.
+// 16-byte piece p sits at p ^ swz(r), which spreads the rows that one read pass covers over the banks
+// (counters: the LDS is active 25-36 % of a launch, 30-43 % of that are bank conflicts, of the reads and the
+// staged output together).
 // x is the MFMA's first source, so a lane holds four consecutive columns of one output row; the tile
 // is packed to 16 bits, staged through LDS and stored as whole 256-byte rows.
 //
